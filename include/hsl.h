@@ -50,9 +50,10 @@ int hsl_abi_version(void);
 const char* hsl_last_error(void);
 
 /* Recurrent-path selection: 0 = automatic (persistent kernels where the shape
- * fits on chip, else one launch per time step), 1 = always per-step,
- * 2 = persistent only (HSL_ERR_UNSUPPORTED if it does not fit).  Returns the
- * previous value.  Process-wide. */
+ * fits on chip in up to four launches over the batch, else one launch per time
+ * step), 1 = always per-step, 2 = persistent in one launch only
+ * (HSL_ERR_UNSUPPORTED if it does not fit).  Returns the previous value.
+ * Process-wide. */
 int hsl_set_recurrent_path(int mode);
 /* Bound, in microseconds, on any wait a persistent kernel does for another
  * workgroup (default 2,000,000).  On expiry the kernel stops and raises the

@@ -618,6 +618,7 @@ struct PFwdArgs {
   unsigned long long* hello;  // [NG][NWMAX]
   int* err;
   int T, B, H, Hp, NG, NGX, Bg, NW;
+  int g0, ng;        // groups of this launch: g0 .. g0 + ng - 1 of the NG
   int device_scope;  // 1: never use the XCD-local stores
   long long spin;
   // input-projection waves (launches with 512 threads; gih is then unused)
@@ -1124,8 +1125,8 @@ __global__ __launch_bounds__(XP ? 512 : 256, 1) void rec_fwd_persistent(PFwdArgs
   __shared__ int abort_flag;
   extern __shared__ char dyn_lds[];  // keeps one workgroup per CU; xin (XP), the saves, the W_hh staging
   XinBuf* const xin = reinterpret_cast<XinBuf*>(dyn_lds);
-  const int grp = blockIdx.x % p.NGX, wg = blockIdx.x / p.NGX;
-  if (grp >= p.NG) return;  // unused XCD slot (groups are padded to a multiple of 8)
+  const int lg = blockIdx.x % p.NGX, grp = p.g0 + lg, wg = blockIdx.x / p.NGX;
+  if (lg >= p.ng) return;  // unused XCD slot (groups are padded to a multiple of 8)
   if (threadIdx.x == 0) abort_flag = 0;
   if (threadIdx.x < 4) step_flags()[threadIdx.x] = 0;  // steps whose h wave q has published
   const bool fast = agree_placement(p.hello + (size_t)grp * (HP / kUnits), wg, p.NW, p.spin, &abort_flag, p.err) &&
@@ -1184,6 +1185,7 @@ struct PBwdArgs {
   unsigned long long* hello;  // [NG][NWMAX]
   int* err;
   int T, B, H, Hp, NG, NGX, Bg, NW;
+  int g0, ng;  // groups of this launch: g0 .. g0 + ng - 1 of the NG
   int device_scope;
   long long spin;
   // weight-gradient waves (launches with 512 threads): fp32 partial sums of
@@ -1778,17 +1780,17 @@ __device__ __forceinline__ bool rec_bwd_wgrad_win(const PBwdArgs& p, int grp, in
     const int g = tile_g(c), sub = tile_sub(c);
     f4 xa[4] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
     // piece product i of the four row tiles in turn: four independent accumulators
-    // between dependent products
+    // between dependent products.  The six products go to a zeroed partial that is added to
+    // the long running sum once: adding each to it directly rounded that sum six times a
+    // window (relative error of dW_hh at T = 256: 5.2e-7, now 1.9e-7; same step time)
 #pragma unroll
     for (int i = 5; i >= 0; --i)
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) {
-        if (c < NH)
-          acch[g][sub][rt] = mfma16_bf16(a[rt][kPa[i]], bp[kPb[i]], acch[g][sub][rt]);
-        else
-          xa[rt] = mfma16_bf16(a[rt][kPa[i]], bp[kPb[i]], xa[rt]);
-      }
-    if (c >= NH) {  // the window's dW_ih tile into the fp64 copy
+      for (int rt = 0; rt < 4; ++rt) xa[rt] = mfma16_bf16(a[rt][kPa[i]], bp[kPb[i]], xa[rt]);
+    if (c < NH) {
+#pragma unroll
+      for (int rt = 0; rt < 4; ++rt) acch[g][sub][rt] = acch[g][sub][rt] + xa[rt];
+    } else {  // the window's dW_ih tile into the fp64 copy
       double* const xl = xacc + (4 * (ol >> 4)) * 256 + (w + 4 * g) * 32 + 16 * sub + (ol & 15);
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt)
@@ -1981,8 +1983,8 @@ __global__ __launch_bounds__(XT >= 0 ? 512 : 256, 1) void rec_bwd_persistent(PBw
   constexpr bool GW = XT >= 0;
   __shared__ float dgl[2][4][64 + 4];  // [step parity][batch slot][gate row]
   __shared__ int abort_flag;
-  const int grp = blockIdx.x % p.NGX, wg = blockIdx.x / p.NGX;
-  if (grp >= p.NG) return;
+  const int lg = blockIdx.x % p.NGX, grp = p.g0 + lg, wg = blockIdx.x / p.NGX;
+  if (lg >= p.ng) return;
   if (threadIdx.x == 0) abort_flag = 0;
   if (threadIdx.x < 4) step_flags()[threadIdx.x] = 0;  // steps whose products wave q has issued
   const bool fast = agree_placement(p.hello + (size_t)grp * NWMAX, wg, p.NW, p.spin, &abort_flag, p.err) &&
@@ -2033,6 +2035,7 @@ __global__ __launch_bounds__(XT >= 0 ? 512 : 256, 1) void rec_bwd_persistent(PBw
 struct PersistentPlan {
   bool ok = false;
   int KQ = 0, Hp = 0, NG = 0, NGX = 0, Bg = 0, NW = 0, grid = 0;
+  int launches = 1, gpl = 0;  // launches of gpl groups each (the last may have fewer)
   int XT = -1;  // backward: -1 no weight-gradient waves, 0 dW_hh only, 2 dW_hh and dW_ih
   bool XP = false;  // forward: input projection inside the kernel (512 threads)
   bool XS = false;  // with XP: its products on split bf16 pieces
@@ -2107,6 +2110,16 @@ int bwd_resident(int xt, bool ws, int* occ) {
   return ws ? bwd_resident_ws<KQ, true>(xt, occ) : bwd_resident_ws<KQ, false>(xt, occ);
 }
 
+// Launches a batch may be split into before the per-step path takes over.  One launch costs
+// about 1.5 us per step forward and 2.6 us backward whatever its group count; the per-step
+// path's cost grows slowly with B.  us per step (forward, backward) at T = 64, D = 256,
+// launches against per step:
+//   H = 512: B = 64 (2) 3.5, 5.2 / 8.6, 12.1;  B = 128 (4) 6.9, 10.5 / 8.0, 15.5;
+//            B = 192 (6) 10.4, 16.0 / 10.6, 18.8;  B = 256 (8) 13.8, 22.0 / 11.5, 19.9
+//   H = 384: B = 128 (4) 6.5, 9.7 / 7.2, 14.3;  B = 192 (6) 9.7, 14.4 / 8.9, 16.2
+//   H = 256: B = 128 (2) 2.6, 4.0 / 5.8, 10.6;  H = 128: B = 256 (2) 2.2, 3.7 / 5.1, 9.8
+constexpr int kMaxGroupLaunches = 4;
+
 int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
   *pl = PersistentPlan{};
   const int mode = recurrent_path_mode();
@@ -2120,11 +2133,7 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
   p.Hp = 4 * kq;
   p.NG = (B + 3) / 4;
   p.Bg = (B + p.NG - 1) / p.NG;
-  // group g is served by workgroups blockIdx % NGX == g; NGX is a multiple of the XCD
-  // count so that every group sits on one XCD (workgroup i runs on XCD i % 8)
-  p.NGX = (p.NG + di.num_xcds - 1) / di.num_xcds * di.num_xcds;
   p.NW = (H + kUnits - 1) / kUnits;
-  p.grid = p.NGX * p.NW;
   // dW_ih joins the weight-gradient waves when its 32-column tiles fit two per wave
   if (bwd && fused_wgrad_enabled()) p.XT = (D > 0 && D <= 256) ? 2 : 0;
   // the forward's projection waves hold W_ih rows for a quarter of D <= 256 each and read
@@ -2150,9 +2159,20 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
         default: HSL_CHECK(fwd_resident<128>(xp, &occ)); break;
       }
     }
-    // every workgroup must be resident at once: the waits are between workgroups
-    p.ok = occ >= 1 && (long)occ * di.num_cus >= p.grid;
-    if (p.ok || (p.XT < 0 && !p.XP)) break;
+    // every workgroup of a launch must be resident at once: the waits are between them.
+    // The groups never wait for each other, so a batch of more groups than fit runs as
+    // several launches of as equal a number of groups as possible.  Group g0 + i of a launch
+    // is served by workgroups blockIdx % NGX == i; NGX is a multiple of the XCD count so
+    // that every group sits on one XCD (workgroup i runs on XCD i % 8).
+    const int fit = (int)((long)occ * di.num_cus / p.NW / di.num_xcds) * di.num_xcds;
+    if (fit > 0) {
+      p.launches = (p.NG + fit - 1) / fit;
+      p.gpl = (p.NG + p.launches - 1) / p.launches;
+      p.NGX = (p.gpl + di.num_xcds - 1) / di.num_xcds * di.num_xcds;
+      p.grid = p.NGX * p.NW;
+      p.ok = p.launches <= (mode == 2 ? 1 : kMaxGroupLaunches);
+    }
+    if (p.ok || fit > 0 || (p.XT < 0 && !p.XP)) break;
     p.XT = -1;  // retry without the weight-gradient / projection waves
     p.XP = false;
   }
@@ -2584,17 +2604,20 @@ int hsl_rec_fwd(const float* x, const float* h0, const float* c0, const float* w
 
   if (pl.ok) {
     PFwdArgs pa{w.gih, w_hh, b_hh, a, h0, c0, h_save, c_save, gact, tanh_c, w.xbuf, w.hello, w.err,
-                T, B, H, pl.Hp, pl.NG, pl.NGX, pl.Bg, pl.NW, exchange_scope_mode(), spin_timeout_ticks(),
+                T, B, H, pl.Hp, pl.NG, pl.NGX, pl.Bg, pl.NW, 0, 0, exchange_scope_mode(), spin_timeout_ticks(),
                 x, w_ih, b_ih, D};
     const int xp = pl.XP ? (pl.XS ? 2 : 1) : 0;
     const int slot = timing_begin(kTimeRecFwd, s);
-    switch (pl.KQ) {
-      case 16: launch_fwd_persistent<16>(pa, pl.grid, xp, s); break;
-      case 32: launch_fwd_persistent<32>(pa, pl.grid, xp, s); break;
-      case 64: launch_fwd_persistent<64>(pa, pl.grid, xp, s); break;
-      default: launch_fwd_persistent<128>(pa, pl.grid, xp, s); break;
+    for (; pa.g0 < pl.NG; pa.g0 += pl.gpl) {
+      pa.ng = std::min(pl.gpl, pl.NG - pa.g0);
+      switch (pl.KQ) {
+        case 16: launch_fwd_persistent<16>(pa, pl.grid, xp, s); break;
+        case 32: launch_fwd_persistent<32>(pa, pl.grid, xp, s); break;
+        case 64: launch_fwd_persistent<64>(pa, pl.grid, xp, s); break;
+        default: launch_fwd_persistent<128>(pa, pl.grid, xp, s); break;
+      }
+      HSL_HIP(hipGetLastError());
     }
-    HSL_HIP(hipGetLastError());
     timing_end(slot, s);
     note_recurrent_path(2);
     return HSL_OK;
@@ -2664,7 +2687,12 @@ int hsl_rec_fwd_noalloc(const float* x, const float* h0, const float* c0, const 
   const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
   if (pl.XP && !x_aligned) pl.XP = false;
   FwdWs w;
-  const size_t need = carve_fwd(nullptr, 0, T, B, H, fwd_needs(pl, wp, x_aligned), &w);
+  size_t need = carve_fwd(nullptr, 0, T, B, H, fwd_needs(pl, wp, x_aligned), &w);
+  if (pl.launches > 1) {  // a batch beyond one launch is held to the per-step path's buffers
+    FwdNeeds step;
+    step.xch = step.wide = false;
+    need = std::max(need, carve_fwd(nullptr, 0, T, B, H, step, &w));
+  }
   if (need > kNoAllocScratchBytes)
     return fail(HSL_ERR_UNSUPPORTED,
                 "hsl_rec_fwd_noalloc: T=%d B=%d D=%d H=%d needs %zu bytes of scratch, more than the %zu bytes of "
@@ -2747,18 +2775,21 @@ int hsl_rec_bwd(const float* dout, const float* dh_n, const float* dc_n, const f
     HSL_CHECK(zero_words(reinterpret_cast<unsigned long long*>(w.err), 32, s));
   if (pl.ok) {
     PBwdArgs pa{dout, dh_n, dc_n, c_save, gact, tanh_c, w_hh, a, w.dgates, w.db_part, dh0, dc0, w.pbuf, w.hello,
-                w.err, T, B, H, pl.Hp, pl.NG, pl.NGX, pl.Bg, pl.NW, exchange_scope_mode(), spin_timeout_ticks(),
+                w.err, T, B, H, pl.Hp, pl.NG, pl.NGX, pl.Bg, pl.NW, 0, 0, exchange_scope_mode(), spin_timeout_ticks(),
                 h_save, x, wph, fused_ih ? wpx : nullptr, D, wts,
                 // dgates feed the GEMMs for whatever the kernel does not produce itself
                 (!fused_ih || dx != nullptr) ? 1 : 0};
     const int slot = timing_begin(kTimeRecBwd, s);
-    switch (pl.KQ) {
-      case 16: launch_bwd_persistent<16>(pa, pl.grid, pl.XT, pl.WS, s); break;
-      case 32: launch_bwd_persistent<32>(pa, pl.grid, pl.XT, pl.WS, s); break;
-      case 64: launch_bwd_persistent<64>(pa, pl.grid, pl.XT, pl.WS, s); break;
-      default: launch_bwd_persistent<128>(pa, pl.grid, pl.XT, pl.WS, s); break;
+    for (; pa.g0 < pl.NG; pa.g0 += pl.gpl) {
+      pa.ng = std::min(pl.gpl, pl.NG - pa.g0);
+      switch (pl.KQ) {
+        case 16: launch_bwd_persistent<16>(pa, pl.grid, pl.XT, pl.WS, s); break;
+        case 32: launch_bwd_persistent<32>(pa, pl.grid, pl.XT, pl.WS, s); break;
+        case 64: launch_bwd_persistent<64>(pa, pl.grid, pl.XT, pl.WS, s); break;
+        default: launch_bwd_persistent<128>(pa, pl.grid, pl.XT, pl.WS, s); break;
+      }
+      HSL_HIP(hipGetLastError());
     }
-    HSL_HIP(hipGetLastError());
     timing_end(slot, s);
     note_recurrent_path(2);
     note_backward_fused(fused_ih ? 2 : fused ? 1 : 0);

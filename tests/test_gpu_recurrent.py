@@ -154,6 +154,22 @@ def test_device_scope_exchange(dev, shape):
     check(*shape, dev, 2, a=[0.6, 0.2, 0.9, 0.4])
 
 
+@pytest.mark.parametrize("T,B,D,H", [(9, 33, 20, 512),    # 9 groups: launches of 5 and 4
+                                     (3, 128, 16, 512),   # the most launches: 4 of 8 groups
+                                     (9, 66, 270, 300),   # D > 256: separate dW_ih, dgates of both launches
+                                     (2, 261, 12, 20)])   # 66 groups of two workgroups, a last group of one row
+def test_batch_over_several_launches(dev, T, B, D, H):
+    """A batch of more groups than the chip holds at once runs as several launches of the
+    persistent kernels, each over its own groups of the same buffers (path 2); a fifth launch
+    would take the per-step path."""
+    check(T, B, D, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=True, fwd_path=2)
+    assert prlstm_amd.last_recurrent_path() == 2
+
+
+def test_batch_beyond_the_launches(dev):
+    check(2, 129, 16, 512, dev, 0, a=[0.3, 0.5, 0.1, 0.2], fwd_path=1)
+
+
 def test_config2_nonlinear_a(dev):
     """configs[2] variant: a ~ U(0, 0.5) drawn right after init."""
     torch.manual_seed(0)
