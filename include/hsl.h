@@ -51,8 +51,8 @@ const char* hsl_last_error(void);
 
 /* Recurrent-path selection: 0 = automatic (persistent kernels where the shape
  * fits on chip in up to four launches over the batch, else one launch per time
- * step), 1 = always per-step, 2 = persistent in one launch only
- * (HSL_ERR_UNSUPPORTED if it does not fit).  Returns the previous value.
+ * step), 1 = always per-step, 2 = persistent in one launch of a whole width only
+ * (H <= 512, or 1024 or 2048 with B <= 32; else HSL_ERR_UNSUPPORTED).  Returns the previous value.
  * Process-wide. */
 int hsl_set_recurrent_path(int mode);
 /* Bound, in microseconds, on any wait a persistent kernel does for another
@@ -85,7 +85,7 @@ int hsl_set_split_products(int on);
 /* Which path the last hsl_rec_fwd / hsl_rec_bwd in this process (on any host
  * thread; autograd runs the backward on its own thread) used: 1 = per-step,
  * 2 = persistent, 3 = the persistent kernels that hold W_hh in the registers of
- * 256 workgroups (H = 1024 or 2048, B <= 32). */
+ * 256 workgroups (512 < H <= 2048). */
 int hsl_last_recurrent_path(void);
 /* Whether the last hsl_rec_bwd (in this process, on any thread) accumulated the
  * weight gradients inside the persistent kernel: 0 = no (separate GEMMs), 1 = dW_hh,

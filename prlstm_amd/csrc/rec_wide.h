@@ -1,6 +1,7 @@
-// Persistent recurrent kernels for a large hidden size, H = 32 U with U = 64 (H = 2048,
-// configs[3]) or U = 32 (H = 1024, the reference's published T64 B32 D512 H1024 shape),
-// B <= 32.  Included by recurrent.hip: they share that file's hand-off helpers and its
+// Persistent recurrent kernels for a large hidden size, widths 32 U with U = 64 (2048,
+// configs[3]) or U = 32 (1024, the reference's published T64 B32 D512 H1024 shape).  A hidden
+// size below its width runs on PAD instances, whose units past H read and store nothing but
+// take part in every hand-off (separate instances: the conditions cost configs[3] 3%).  A launch runs at most 32 batch rows.  Included by recurrent.hip: they share that file's hand-off helpers and its
 // device error word.  This file holds what the wide forward (rec_wide_fwd.h) and the
 // backwards share -- the grid, the hand-off buffers and their access helpers, the slot
 // rotation, the 16x16x4 product helper -- and the two-chain backward run at H = 2048 (the
@@ -115,8 +116,8 @@ __device__ __forceinline__ void wide_drain16(f4 (&acc)[RT][2]) {
 }
 
 // ---------------------------------------------------------------------------------
-// Persistent recurrent backward for H = 32 U, B <= 32, run for U = 64 (H = 2048, configs[3];
-// H = 1024 runs the single-chain form of rec_wide_bwd32.h): the mirror of the wide forward
+// Persistent recurrent backward for H <= 32 U, at most 32 batch rows, run for U = 64 (H > 1024;
+// smaller H runs the single-chain form of rec_wide_bwd32.h): the mirror of the wide forward
 // in rec_wide_fwd.h (_torch.py:133-150:
 // dh_t = dout_t + dg_{t+1} W_s, then the cell backward).  Workgroup (x, c), blockIdx =
 // x + 8 c, sits on XCD x and holds W_hh's 16U gate rows of units [4U x, +4U) (unit-
@@ -193,12 +194,12 @@ struct WBwdArgs {
   float* inbox;         // [3 slots][2 chains][256 workgroups][INBOX]
   unsigned long long* hello;  // [8][32]
   int* err;
-  int T, B, H;
+  int T, B, H, nb;   // nb: batch rows of this launch (the pointers are at its first row; B strides)
   int device_scope;
   long long spin;
 };
 
-template <int U, bool FAST>
+template <int U, bool FAST, bool PAD>
 __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int c, float* red, float* gst,
                                                   int& abort_flag) {
   using S = WideBShape<U>;
@@ -208,7 +209,8 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
   const int ubase = 4 * U * x;  // first unit of the XCD's rows
-  const int nch = B > 16 ? 2 : 1;
+  const int nb = p.nb;
+  const int nch = nb > 16 ? 2 : 1;
 
   // W_hh^T block of this wave: group j, k-step e, column tile ct -> row 4U w + 4 (4j + e) +
   // l/16 (unit ubase + U w + 4j + e, gate l/16), column U c + 16 ct + l%16; unscaled, a
@@ -216,6 +218,17 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
   float wreg[NQ][4][CT];
   {
     const float* const wb = p.w_hh + ((size_t)lq * H + ubase + U * w) * H + U * c + l16;
+    // PAD: units and columns past H are read clamped and held as 0; the unit is wave-uniform,
+    // so its row is a scalar base and the lane's gate and column one offset
+    const float* const w_hh = p.w_hh;
+    unsigned off[PAD ? CT : 1], keep[PAD ? CT : 1];
+    if constexpr (PAD) {
+#pragma unroll
+      for (int ct = 0; ct < CT; ++ct) {
+        keep[ct] = U * c + 16 * ct + l16 < H ? ~0u : 0u;
+        off[ct] = 4u * ((unsigned)lq * H * H + min(U * c + 16 * ct + l16, H - 1));
+      }
+    }
 #pragma unroll
     for (int j8 = 0; j8 < NQ; j8 += 4) {
 #pragma unroll
@@ -223,7 +236,15 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-          for (int ct = 0; ct < CT; ++ct) wreg[j][e][ct] = wb[(size_t)(4 * j + e) * H + 16 * ct];
+          for (int ct = 0; ct < CT; ++ct) {
+            if constexpr (PAD) {
+              const int u = ubase + U * w + 4 * j + e;
+              const unsigned v = __float_as_uint(*byte_at(w_hh + (size_t)min(u, H - 1) * H, off[ct]));
+              wreg[j][e][ct] = __uint_as_float(u < H ? v & keep[ct] : 0u);
+            } else {
+              wreg[j][e][ct] = wb[(size_t)(4 * j + e) * H + 16 * ct];
+            }
+          }
 #pragma unroll
       for (int j = j8; j < j8 + 4; ++j)
 #pragma unroll
@@ -238,14 +259,16 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
   const int rc = tid >> 7, ri = tid & 127;
   const bool reducer = ri < S::REDUCERS;
   const int su = ri >> 4, cb = ri & 15, brow = 16 * rc + cb;
-  const bool c_ok = reducer && brow < B;
   const int unit = ubase + SU * c + su;
+  // a unit past H (u_ok false) waits for and clears its partials as the others do (the slot
+  // rotation rests on it), reads and stores nothing and publishes 0
+  const bool c_ok = reducer && brow < nb, u_ok = c_ok && (!PAD || unit < H);
   float ag[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) ag[g] = p.a[g];
   float dc = 0.f;
   double dbacc[4] = {0.0, 0.0, 0.0, 0.0};
-  if (c_ok && p.dc_n) dc = p.dc_n[(size_t)brow * H + unit];
+  if (u_ok && p.dc_n) dc = p.dc_n[(size_t)brow * H + unit];
   const size_t plane = (size_t)B * H, plane4 = 4 * plane;
   // sender role: thread -> slice c4 of the workgroup's columns, batch row sb of the chain,
   // quad qq of the slice's SU units; the slice goes to reducer (c / 4, 8 (c % 4) + c4)
@@ -315,7 +338,7 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
       // every lane stores, lanes without a partial past the descriptor's end (dropped), so
       // that the store's count in the completion counter does not depend on the lane
       const __amdgpu_buffer_rsrc_t d = wide_rsrc(inbox(k - 1, ch, 0), (size_t)kWideWgs * S::INBOX);
-      const bool mine = sender && 16 * ch + sb < B;
+      const bool mine = sender && 16 * ch + sb < nb;
       const int cq = S::QS * c4 + qq;
       f4 sum = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -334,7 +357,7 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
   auto cell_in = [&](int ch, int k, CellIn& in) {
     in = CellIn{0.f, 0.f, 0.f, 0.f, f4{0.f, 0.f, 0.f, 0.f}};
     if (rc == ch && k < T) {
-      const size_t ec = c_ok ? (size_t)brow * H + unit : 0, tp = (size_t)(T - 1 - k) * plane + ec;
+      const size_t ec = u_ok ? (size_t)brow * H + unit : 0, tp = (size_t)(T - 1 - k) * plane + ec;
       in.dout = p.dout[tp];
       in.ga = *reinterpret_cast<const f4*>(p.gact + tp * 4);
       in.c = p.c_save[tp];
@@ -371,7 +394,7 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
       for (int sx = 1; sx < 8; ++sx) dsum += __uint_as_float(v[sx]);
     }
     if (k == T) {  // dh of h0, the carry into c0, the bias partials
-      if (mine && c_ok) {
+      if (mine && u_ok) {
         const size_t e = (size_t)brow * H + unit;
         if (p.dh0) p.dh0[e] = dsum;
         if (p.dc0) p.dc0[e] = dc;
@@ -382,7 +405,7 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
     }
     const int t = T - 1 - k;
     float d[4] = {0.f, 0.f, 0.f, 0.f};
-    if (mine && c_ok) {
+    if (mine && u_ok) {
       const float dh = (k > 0 ? dsum : in.dhn) + in.dout;
       cell_bwd(dh, dc, in.c, in.ga[0], in.ga[1], in.ga[2], in.ga[3], in.tc, d);
       float* const dg = p.dgates + (size_t)t * plane4 + (size_t)brow * 4 * H + unit;
@@ -396,7 +419,7 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
     float* const gs = gst + ch * S::GROUP;
     if (mine && reducer) {
 #pragma unroll
-      for (int g = 0; g < 4; ++g) gs[256 * (su >> 2) + 4 * (16 * g + cb) + (su & 3)] = c_ok ? canon_nan(ag[g] * d[g]) : 0.f;
+      for (int g = 0; g < 4; ++g) gs[256 * (su >> 2) + 4 * (16 * g + cb) + (su & 3)] = u_ok ? canon_nan(ag[g] * d[g]) : 0.f;
     }
     lds_barrier();
     if (abort_flag) return false;
@@ -469,11 +492,11 @@ __device__ __forceinline__ void rec_bwd_wide_body(const WBwdArgs& p, int x, int 
 // After an abort the reducer lanes set what they own to NaN: dgates of their unit and batch
 // row at every step, the bias partials, and dh0 / dc0.
 template <int U>
-__device__ void poison_wide_bwd(const WBwdArgs& p, int x, int c) {
+__device__ __forceinline__ void poison_wide_bwd(const WBwdArgs& p, int x, int c) {
   using S = WideBShape<U>;
   const int tid = threadIdx.x, ri = tid & 127, su = ri >> 4, brow = 16 * (tid >> 7) + (ri & 15);
-  if (ri >= S::REDUCERS || brow >= p.B) return;
   const int unit = 4 * U * x + S::SU * c + su, H = p.H;
+  if (ri >= S::REDUCERS || brow >= p.nb || unit >= H) return;
   const float nan = __uint_as_float(0x7FC00000u);
   const size_t e = (size_t)brow * H + unit;
   if (p.dh0) p.dh0[e] = nan;
@@ -483,7 +506,7 @@ __device__ void poison_wide_bwd(const WBwdArgs& p, int x, int c) {
     for (int g = 0; g < 4; ++g) p.dgates[((size_t)t * p.B + brow) * 4 * H + g * H + unit] = nan;
 }
 
-template <int U>
+template <int U, bool PAD>
 __global__ __launch_bounds__(256, 1) void rec_bwd_wide(WBwdArgs p) {
   using S = WideBShape<U>;
   extern __shared__ float wide_lds[];  // per chain: wave partials; then per chain the dg group (padded: one workgroup per CU)
@@ -495,9 +518,9 @@ __global__ __launch_bounds__(256, 1) void rec_bwd_wide(WBwdArgs p) {
                     !p.device_scope;
   if (!abort_flag) {
     if (fast)
-      rec_bwd_wide_body<U, true>(p, x, c, wide_lds, wide_lds + 2 * 4 * S::RED, abort_flag);
+      rec_bwd_wide_body<U, true, PAD>(p, x, c, wide_lds, wide_lds + 2 * 4 * S::RED, abort_flag);
     else
-      rec_bwd_wide_body<U, false>(p, x, c, wide_lds, wide_lds + 2 * 4 * S::RED, abort_flag);
+      rec_bwd_wide_body<U, false, PAD>(p, x, c, wide_lds, wide_lds + 2 * 4 * S::RED, abort_flag);
   }
   lds_barrier();
   if (abort_flag) poison_wide_bwd<U>(p, x, c);

@@ -1,4 +1,4 @@
-// Single-chain persistent recurrent backward for H = 1024 (U = 32), B <= 32.  Included by
+// Single-chain persistent recurrent backward for 512 < H <= 1024 (U = 32), at most 32 batch rows.  Included by
 // recurrent.hip after rec_wide.h, whose grid, hand-off helpers, slot rotation and argument
 // block it uses; it reads the same buffers as the two-chain backward there, laid out for one
 // chain of 32 batch rows.  At H = 1024 a step's products are a quarter of those at H = 2048
@@ -84,12 +84,12 @@ __device__ __forceinline__ unsigned wideb1_pos(int rho, int b) {
   return 128u * U * w + 256u * (i >> 2) + 4u * l + (i & 3);
 }
 
-template <int U, bool FAST>
+template <int U, bool FAST, bool PAD>
 __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int c, float* red, float* gst,
                                                   int& abort_flag) {
   using S = WideB1Shape<U>;
   constexpr int CT = S::CT, SU = S::SU;
-  const int T = p.T, B = p.B, H = p.H;
+  const int T = p.T, B = p.B, H = p.H, nb = p.nb;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hb = lane >> 5, l32 = lane & 31;
@@ -105,10 +105,15 @@ __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int
     for (int i4 = i8; i4 < i8 + 4; ++i4)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int rho = S::WROWS * w + 2 * (4 * i4 + e) + hb;
-        const float* row = p.w_hh + ((size_t)(rho & 3) * H + ubase + (rho >> 2)) * H + U * c + l32;
+        // units and columns past H (a padded width) are read clamped and held as 0
+        const int rho = S::WROWS * w + 2 * (4 * i4 + e) + hb, u = ubase + (rho >> 2);
+        const float* row = p.w_hh + ((size_t)(rho & 3) * H + (PAD ? min(u, H - 1) : u)) * H;
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) wreg[i4][e][ct] = row[32 * ct];
+        for (int ct = 0; ct < CT; ++ct) {
+          const int cc = U * c + 32 * ct + l32;
+          const float v = row[PAD ? min(cc, H - 1) : cc];
+          wreg[i4][e][ct] = !PAD || (u < H && cc < H) ? v : 0.f;
+        }
       }
 #pragma unroll
     for (int i4 = i8; i4 < i8 + 4; ++i4)
@@ -122,16 +127,18 @@ __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int
   // units ubase + SU c + su), batch cb
   const int su = tid >> 5, cb = tid & 31;
   const bool reducer = tid < S::REDUCERS;
-  const bool c_ok = reducer && cb < B;
   const int unit = ubase + SU * c + su;
+  // a unit past H (u_ok false) waits for and clears its partials as the others do (the slot
+  // rotation rests on it), reads and stores nothing and publishes 0
+  const bool c_ok = reducer && cb < nb, u_ok = c_ok && (!PAD || unit < H);
   float ag[4];
 #pragma unroll
   for (int g = 0; g < 4; ++g) ag[g] = p.a[g];
   float dc = 0.f;
   double dbacc[4] = {0.0, 0.0, 0.0, 0.0};
-  if (c_ok && p.dc_n) dc = p.dc_n[(size_t)cb * H + unit];
+  if (u_ok && p.dc_n) dc = p.dc_n[(size_t)cb * H + unit];
   const size_t plane = (size_t)B * H, plane4 = 4 * plane;
-  const bool h_ok = l32 < B;
+  const bool h_ok = l32 < nb;
   // broadcast buffer of this XCD; this workgroup's group in it
   const size_t bslot = (size_t)kWideXcds * S::ROWS * 32;
   float* const bx = p.dgbuf + (size_t)x * S::ROWS * 32;
@@ -147,7 +154,7 @@ __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int
     float in_do = 0.f, in_c = 0.f, in_tc = 0.f, in_dhn = 0.f;
     f4 in_ga = f4{0.f, 0.f, 0.f, 0.f};
     if (reducer && k < T) {
-      const size_t ec = c_ok ? (size_t)cb * H + unit : 0, tp = (size_t)t * plane + ec;
+      const size_t ec = u_ok ? (size_t)cb * H + unit : 0, tp = (size_t)t * plane + ec;
       in_do = p.dout[tp];
       in_ga = *reinterpret_cast<const f4*>(p.gact + tp * 4);
       in_c = p.c_save[tp];
@@ -207,7 +214,7 @@ __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int
               wide_partial1(acc, q);
       lds_barrier();
       if (abort_flag) return;
-      if (sb < B) {
+      if (sb < nb) {
         const __amdgpu_buffer_rsrc_t d =
             wide_rsrc(p.inbox + (size_t)((k - 1) % kWidePSlots) * islot, (size_t)kWideWgs * S::INBOX);
 #pragma unroll
@@ -247,7 +254,7 @@ __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int
       }
     }
     if (k == T) {  // dh of h0, the carry into c0, the bias partials
-      if (c_ok) {
+      if (u_ok) {
         if (p.dh0) p.dh0[(size_t)cb * H + unit] = dsum;
         if (p.dc0) p.dc0[(size_t)cb * H + unit] = dc;
 #pragma unroll
@@ -257,7 +264,7 @@ __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int
     }
     // ---- 3b. cell backward of step t, dgates_t, the broadcast of a_g dg_t ---------------
     float d[4] = {0.f, 0.f, 0.f, 0.f};
-    if (c_ok) {
+    if (u_ok) {
       const float dh = (k > 0 ? dsum : in_dhn) + in_do;
       cell_bwd(dh, dc, in_c, in_ga[0], in_ga[1], in_ga[2], in_ga[3], in_tc, d);
       float* const dg = p.dgates + (size_t)t * plane4 + (size_t)cb * 4 * H + unit;
@@ -272,7 +279,7 @@ __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int
     if (reducer) {
 #pragma unroll
       for (int g = 0; g < 4; ++g)
-        gst[wideb1_pos<U>(4 * (SU * c + su) + g, cb) - (unsigned)S::GROUP * c] = c_ok ? canon_nan(ag[g] * d[g]) : 0.f;
+        gst[wideb1_pos<U>(4 * (SU * c + su) + g, cb) - (unsigned)S::GROUP * c] = u_ok ? canon_nan(ag[g] * d[g]) : 0.f;
     }
     lds_barrier();
     if (abort_flag) return;
@@ -292,11 +299,11 @@ __device__ __forceinline__ void rec_bwd_wide1_body(const WBwdArgs& p, int x, int
 // After an abort the reducer lanes set what they own to NaN: dgates of their unit and batch
 // row at every step, the bias partials, and dh0 / dc0.
 template <int U>
-__device__ void poison_wide_bwd1(const WBwdArgs& p, int x, int c) {
+__device__ __forceinline__ void poison_wide_bwd1(const WBwdArgs& p, int x, int c) {
   using S = WideB1Shape<U>;
   const int tid = threadIdx.x, su = tid >> 5, cb = tid & 31;
-  if (tid >= S::REDUCERS || cb >= p.B) return;
   const int unit = 4 * U * x + S::SU * c + su, H = p.H;
+  if (tid >= S::REDUCERS || cb >= p.nb || unit >= H) return;
   const float nan = __uint_as_float(0x7FC00000u);
   const size_t e = (size_t)cb * H + unit;
   if (p.dh0) p.dh0[e] = nan;
@@ -306,7 +313,7 @@ __device__ void poison_wide_bwd1(const WBwdArgs& p, int x, int c) {
     for (int g = 0; g < 4; ++g) p.dgates[((size_t)t * p.B + cb) * 4 * H + g * H + unit] = nan;
 }
 
-template <int U>
+template <int U, bool PAD>
 __global__ __launch_bounds__(256, 1) void rec_bwd_wide1(WBwdArgs p) {
   using S = WideB1Shape<U>;
   extern __shared__ float wide_lds[];  // wave partials, then the gathered dg group (padded: one workgroup per CU)
@@ -318,9 +325,9 @@ __global__ __launch_bounds__(256, 1) void rec_bwd_wide1(WBwdArgs p) {
                     !p.device_scope;
   if (!abort_flag) {
     if (fast)
-      rec_bwd_wide1_body<U, true>(p, x, c, wide_lds, wide_lds + 4 * S::RED, abort_flag);
+      rec_bwd_wide1_body<U, true, PAD>(p, x, c, wide_lds, wide_lds + 4 * S::RED, abort_flag);
     else
-      rec_bwd_wide1_body<U, false>(p, x, c, wide_lds, wide_lds + 4 * S::RED, abort_flag);
+      rec_bwd_wide1_body<U, false, PAD>(p, x, c, wide_lds, wide_lds + 4 * S::RED, abort_flag);
   }
   lds_barrier();
   if (abort_flag) poison_wide_bwd1<U>(p, x, c);

@@ -1,5 +1,5 @@
-// Persistent recurrent forward for H = 32 U (U = 64: H = 2048, configs[3]; U = 32:
-// H = 1024), B <= 32, with W_hh resident in the accumulator registers.  Included by
+// Persistent recurrent forward for H = 32 U (U = 64: H = 2048, configs[3]; U = 32: H = 1024)
+// and, as PAD instances, for smaller H on the same width, at most 32 batch rows, with W_hh resident in the accumulator registers.  Included by
 // recurrent.hip after rec_wide.h, whose grid, hand-off helpers and slot rotation it uses.
 //
 // Workgroup (x, r, kb), blockIdx = x + 8 (8 r + kb), sits on XCD x:
@@ -80,11 +80,12 @@ struct WFwdArgs {
   unsigned long long* hello;  // [8][32] placement words
   int* err;
   int T, B, H;
+  int nb;            // batch rows of this launch (the pointers are at its first row; B strides)
   int device_scope;  // 1: partials with device-scope stores too
   long long spin;
 };
 
-template <int U, bool FAST>
+template <int U, bool FAST, bool PAD>
 __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int r, int kb, f4* hs,
                                                    int& abort_flag) {
   using S = WideFShape<U>;
@@ -93,7 +94,8 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lq = lane >> 4;
-  const int nch = B > 16 ? 2 : 1;  // chains with at least one batch row
+  const int nb = p.nb;
+  const int nch = nb > 16 ? 2 : 1;  // chains with at least one batch row
 
   const int ubase = 4 * U * x + U * r;  // first unit of the workgroup's rows
   const int kbase = 4 * U * kb;         // first k (unit) of the workgroup's k block
@@ -102,15 +104,18 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   // lane's quad is 16 consecutive bytes of its row: one load of four rows' 64-byte segments
   // per 16 lanes (4-byte loads of k-steps 4 apart touched 16 rows per instruction and took
   // the first step 31 us after launch at configs[3], against 10 us for the backward's slice)
+  // Rows and k past H (a padded width) are read from clamped addresses and held as 0.
   float wreg[NQ][4][RT];
   {
     const float* rows[RT];
+    bool row_ok[RT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       const int u = ubase + U / 4 * w + 4 * rt + (l16 >> 2);
-      rows[rt] = p.w_hh + ((size_t)(l16 & 3) * H + u) * H + kbase + 4 * lq;
+      row_ok[rt] = !PAD || u < H;
+      rows[rt] = p.w_hh + ((size_t)(l16 & 3) * H + (row_ok[rt] ? u : 0)) * H;
     }
-    const bool w16 = reinterpret_cast<uintptr_t>(p.w_hh) % 16 == 0;  // uniform
+    const bool w16 = H % 4 == 0 && reinterpret_cast<uintptr_t>(p.w_hh) % 16 == 0;  // uniform
 #pragma unroll
     for (int j8 = 0; j8 < NQ; j8 += 4) {
 #pragma unroll
@@ -118,14 +123,15 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           f4 v;
-          if (w16) {
-            v = *reinterpret_cast<const f4*>(rows[rt] + 16 * j);
+          const int k = kbase + 16 * j + 4 * lq;
+          if (w16) {  // k is a multiple of 4, as H is: k < H implies k + 3 < H
+            v = *reinterpret_cast<const f4*>(rows[rt] + (PAD ? min(k, H - 4) : k));
           } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = rows[rt][16 * j + e];
+            for (int e = 0; e < 4; ++e) v[e] = rows[rt][PAD ? min(k + e, H - 1) : k + e];
           }
 #pragma unroll
-          for (int e = 0; e < 4; ++e) wreg[j][e][rt] = v[e];
+          for (int e = 0; e < 4; ++e) wreg[j][e][rt] = row_ok[rt] && (!PAD || k + e < H) ? v[e] : 0.f;
         }
 #pragma unroll
       for (int j = j8; j < j8 + 4; ++j)
@@ -140,12 +146,15 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   // batch row n = ci % 16 of each chain
   const bool cell = lane < S::CPW;
   const int ci = S::CPW * w + lane, su = ci >> 4, cn = ci & 15;
-  const int unit = ubase + SU * kb + su;  // < H
+  // A unit past H takes part in every hand-off as the others do (the slot rotation rests on
+  // each member waiting for its partials), reads and stores nothing and publishes 0.
+  const int unit = ubase + SU * kb + su;
+  const bool u_ok = !PAD || unit < H;
   float ag[4] = {0.f, 0.f, 0.f, 0.f}, bs[4] = {0.f, 0.f, 0.f, 0.f}, c_reg[2] = {0.f, 0.f};
   bool c_ok[2];
 #pragma unroll
-  for (int c = 0; c < 2; ++c) c_ok[c] = cell && 16 * c + cn < B;
-  if (cell) {
+  for (int c = 0; c < 2; ++c) c_ok[c] = cell && 16 * c + cn < nb;
+  if (cell && u_ok) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       ag[g] = p.a[g];
@@ -154,7 +163,7 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   }
 #pragma unroll
   for (int c = 0; c < 2; ++c) {
-    if (c_ok[c]) {
+    if (c_ok[c] && u_ok) {
       const size_t e = (size_t)(16 * c + cn) * H + unit;
       c_reg[c] = p.c0 ? p.c0[e] : 0.f;
       p.h_save[e] = p.h0 ? p.h0[e] : 0.f;
@@ -178,14 +187,15 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   // h0 instead (tin = -1).
   auto recv_h0 = [&](int c) {
     f4* const buf = hs + (size_t)c * NQ * 64;
-    const bool h_ok = 16 * c + l16 < B;
+    const bool h_ok = 16 * c + l16 < nb;
 #pragma unroll
     for (int j = 0; j < BQ; ++j) {
       f4 v = f4{0.f, 0.f, 0.f, 0.f};
       if (h_ok && p.h0) {
-        const float* row = p.h0 + (size_t)(16 * c + l16) * H + kbase + U * w + 4 * lq;
+        const float* row = p.h0 + (size_t)(16 * c + l16) * H;
+        const int k = kbase + U * w + 4 * lq + 16 * j;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = row[16 * j + e];
+        for (int e = 0; e < 4; ++e) v[e] = !PAD || k + e < H ? row[k + e] : 0.f;
       }
       buf[(w * BQ + j) * 64 + lane] = v;
     }
@@ -195,7 +205,7 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   };
   // Poll loads are issued by every lane, unconditionally: a lane without a value reads
   // from past the end of the buffer (0, never kEmpty).
-  auto recv_off = [&](int c, int j) { return 16 * c + l16 < B ? 256u * j + 4u * lane : (unsigned)S::HB; };
+  auto recv_off = [&](int c, int j) { return 16 * c + l16 < nb ? 256u * j + 4u * lane : (unsigned)S::HB; };
   // recv_issue requests the words (at H = 2048 right after the last products of a phase,
   // so that their latency overlaps the wait of the following send for those products'
   // results), recv_settle polls until none is kEmpty and writes them to LDS
@@ -207,7 +217,7 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   auto recv_settle = [&](int c, int tin, u4v (&q4)[BQ]) -> bool {
     f4* const buf = hs + (size_t)c * NQ * 64;
     const __amdgpu_buffer_rsrc_t src = recv_src(c, tin);
-    const bool h_ok = 16 * c + l16 < B;
+    const bool h_ok = 16 * c + l16 < nb;
     const long long t0 = wall_clock64();
     while (true) {  // all of the lane's groups reloaded while any word is kEmpty
       unsigned m = 0u;
@@ -235,7 +245,7 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   auto load_gin = [&](int c, int t, float (&gin)[4]) {
 #pragma unroll
     for (int gt = 0; gt < 4; ++gt) gin[gt] = 0.f;
-    if (c_ok[c]) {
+    if (c_ok[c] && u_ok) {
       const float* g = p.gih + (size_t)t * plane4 + (size_t)(16 * c + cn) * 4 * H + unit;
 #pragma unroll
       for (int gt = 0; gt < 4; ++gt) gin[gt] = __builtin_nontemporal_load(g + (size_t)gt * H);
@@ -264,7 +274,7 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
   // on the lane)
   auto send = [&](int c, int t, f4 (&acc)[RT][2]) {
     wide_drain16<RT>(acc);
-    const bool mine = 16 * c + l16 < B;
+    const bool mine = 16 * c + l16 < nb;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
       const int ur = U / 4 * w + 4 * rt + lq;  // unit of the row group
@@ -316,13 +326,15 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
         const float tc = tanh_f(cc);
         const float h = act[3] * tc;
         c_reg[c] = cc;
-        hst[c][4 * (16 * (su >> 2) + cn) + (su & 3)] = canon_nan(h);
-        const size_t e = (size_t)(16 * c + cn) * H + unit;
-        __builtin_nontemporal_store(h, p.h_save + (size_t)(t + 1) * plane + e);
-        __builtin_nontemporal_store(cc, p.c_save + (size_t)(t + 1) * plane + e);
-        __builtin_nontemporal_store(tc, p.tanh_c + (size_t)t * plane + e);
-        __builtin_nontemporal_store(f4{act[0], act[1], act[2], act[3]},
-                                    reinterpret_cast<f4*>(p.gact + ((size_t)t * plane + e) * 4));
+        hst[c][4 * (16 * (su >> 2) + cn) + (su & 3)] = u_ok ? canon_nan(h) : 0.f;
+        if (u_ok) {
+          const size_t e = (size_t)(16 * c + cn) * H + unit;
+          __builtin_nontemporal_store(h, p.h_save + (size_t)(t + 1) * plane + e);
+          __builtin_nontemporal_store(cc, p.c_save + (size_t)(t + 1) * plane + e);
+          __builtin_nontemporal_store(tc, p.tanh_c + (size_t)t * plane + e);
+          __builtin_nontemporal_store(f4{act[0], act[1], act[2], act[3]},
+                                      reinterpret_cast<f4*>(p.gact + ((size_t)t * plane + e) * 4));
+        }
       }
     }
     lds_barrier();  // the chain's h values are gathered
@@ -421,11 +433,11 @@ __device__ __forceinline__ void rec_fwd_wide_body(const WFwdArgs& p, int x, int 
 // After an abort the cell lanes set their outputs (rows 0..T of h_save / c_save, the
 // activations of every step) to NaN: lane (unit su, batch row cb) of the workgroup's slice.
 template <int U>
-__device__ void poison_wide_fwd(const WFwdArgs& p, int x, int r, int kb) {
+__device__ __forceinline__ void poison_wide_fwd(const WFwdArgs& p, int x, int r, int kb) {
   constexpr int SU = WideFShape<U>::SU;
   const int tid = threadIdx.x, su = tid >> 5, cb = tid & 31;
-  if (tid >= 32 * SU || cb >= p.B) return;
   const int unit = 4 * U * x + U * r + SU * kb + su;
+  if (tid >= 32 * SU || cb >= p.nb || unit >= p.H) return;
   const float nan = __uint_as_float(0x7FC00000u);
   const size_t plane = (size_t)p.B * p.H, e = (size_t)cb * p.H + unit;
   for (int t = 0; t <= p.T; ++t) {
@@ -438,7 +450,7 @@ __device__ void poison_wide_fwd(const WFwdArgs& p, int x, int r, int kb) {
   }
 }
 
-template <int U>
+template <int U, bool PAD>
 __global__ __launch_bounds__(256, 1) void rec_fwd_wide(WFwdArgs p) {
   extern __shared__ f4 wide_hs[];  // one h buffer per chain (sized to keep one workgroup per CU)
   __shared__ int abort_flag;
@@ -450,9 +462,9 @@ __global__ __launch_bounds__(256, 1) void rec_fwd_wide(WFwdArgs p) {
                     !p.device_scope;
   if (!abort_flag) {
     if (fast)
-      rec_fwd_wide_body<U, true>(p, x, r, kb, wide_hs, abort_flag);
+      rec_fwd_wide_body<U, true, PAD>(p, x, r, kb, wide_hs, abort_flag);
     else
-      rec_fwd_wide_body<U, false>(p, x, r, kb, wide_hs, abort_flag);
+      rec_fwd_wide_body<U, false, PAD>(p, x, r, kb, wide_hs, abort_flag);
   }
   lds_barrier();
   if (abort_flag) poison_wide_fwd<U>(p, x, r, kb);

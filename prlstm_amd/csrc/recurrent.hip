@@ -1682,7 +1682,7 @@ __device__ __forceinline__ bool for_steps(F&& f) {
   }
 }
 
-template <int KQ, int XT>
+template <int KQ, int XT, bool WSUM>
 __device__ __forceinline__ bool rec_bwd_wgrad_win(const PBwdArgs& p, int grp, int wg, float (&dgl)[2][4][68],
                                                   char* lds, int& abort_flag) {
   constexpr int HT = KQ >= 32 ? KQ / 32 : 1;  // h column groups of 32 per wave (4*KQ >= H)
@@ -1780,17 +1780,21 @@ __device__ __forceinline__ bool rec_bwd_wgrad_win(const PBwdArgs& p, int grp, in
     const int g = tile_g(c), sub = tile_sub(c);
     f4 xa[4] = {f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}, f4{0.f, 0.f, 0.f, 0.f}};
     // piece product i of the four row tiles in turn: four independent accumulators
-    // between dependent products.  The six products go to a zeroed partial that is added to
-    // the long running sum once: adding each to it directly rounded that sum six times a
-    // window (relative error of dW_hh at T = 256: 5.2e-7, now 1.9e-7; same step time)
+    // between dependent products.  WSUM: a window's six products go to a zeroed partial that
+    // is added to the long running sum once; adding each to it directly rounds that sum six
+    // times a window (relative error of dW_hh at T = 256: 5.2e-7 against 1.9e-7)
 #pragma unroll
     for (int i = 5; i >= 0; --i)
 #pragma unroll
-      for (int rt = 0; rt < 4; ++rt) xa[rt] = mfma16_bf16(a[rt][kPa[i]], bp[kPb[i]], xa[rt]);
-    if (c < NH) {
+      for (int rt = 0; rt < 4; ++rt) {
+        f4& sum = c < NH && !WSUM ? acch[g][sub][rt] : xa[rt];
+        sum = mfma16_bf16(a[rt][kPa[i]], bp[kPb[i]], sum);
+      }
+    if (WSUM && c < NH) {
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt) acch[g][sub][rt] = acch[g][sub][rt] + xa[rt];
-    } else {  // the window's dW_ih tile into the fp64 copy
+    }
+    if (c >= NH) {  // the window's dW_ih tile into the fp64 copy
       double* const xl = xacc + (4 * (ol >> 4)) * 256 + (w + 4 * g) * 32 + 16 * sub + (ol & 15);
 #pragma unroll
       for (int rt = 0; rt < 4; ++rt)
@@ -1973,11 +1977,11 @@ __device__ void poison_wgrad(const PBwdArgs& p, int grp, int wg) {
 
 // XT < 0: 256 threads, recurrent waves only (weight gradients by separate GEMMs).
 // XT >= 0: 512 threads; waves 4-7 accumulate dW_hh_s and, when XT > 0, dW_ih, on split
-// bf16 products (WS, rec_bwd_wgrad_win) or on the fp32 instruction (rec_bwd_wgrad), as
-// hsl_set_split_products selects.
+// bf16 products (WS > 0, rec_bwd_wgrad_win) or on the fp32 instruction (rec_bwd_wgrad), as
+// hsl_set_split_products selects; WS = 2 sums each window's products first.
 // As in the forward, every wave ends with one more workgroup barrier and then poisons
 // its outputs if any wave of the workgroup gave up a wait.
-template <int KQ, int XT, bool WS>
+template <int KQ, int XT, int WS>
 __global__ __launch_bounds__(XT >= 0 ? 512 : 256, 1) void rec_bwd_persistent(PBwdArgs p) {
   constexpr int NWMAX = 4 * KQ / kUnits;
   constexpr bool GW = XT >= 0;
@@ -1997,9 +2001,9 @@ __global__ __launch_bounds__(XT >= 0 ? 512 : 256, 1) void rec_bwd_persistent(PBw
         // [64][256] fp64 dW_ih accumulator (XT > 0), then the bf16 A operands of two
         // windows (dynamic LDS)
         extern __shared__ double xacc[];
-        if constexpr (WS)
-          passed_final =
-              rec_bwd_wgrad_win<KQ, (XT > 0 ? XT : 0)>(p, grp, wg, dgl, reinterpret_cast<char*>(xacc), abort_flag);
+        if constexpr (WS > 0)
+          passed_final = rec_bwd_wgrad_win<KQ, (XT > 0 ? XT : 0), WS == 2>(
+              p, grp, wg, dgl, reinterpret_cast<char*>(xacc), abort_flag);
         else
           rec_bwd_wgrad<KQ, (XT > 0 ? XT : 0)>(p, grp, wg, dgl, xacc, abort_flag);
       } else {
@@ -2039,7 +2043,7 @@ struct PersistentPlan {
   int XT = -1;  // backward: -1 no weight-gradient waves, 0 dW_hh only, 2 dW_hh and dW_ih
   bool XP = false;  // forward: input projection inside the kernel (512 threads)
   bool XS = false;  // with XP: its products on split bf16 pieces
-  bool WS = true;   // backward with XT >= 0: weight-gradient products on split bf16 pieces
+  int WS = 2;  // backward with XT >= 0: weight-gradient products on split bf16 pieces (0: fp32 products)
 };
 
 int pick_kq(int H) {
@@ -2085,12 +2089,18 @@ int fwd_resident(int xp, int* occ) {
   }
 }
 
-template <int KQ, bool WS>
+// One launch at KQ = 128 adds the weight-gradient products straight to the long sums (WS = 1):
+// there the additions of the window sums lengthen the launch by 0.6% (519 -> 522 us at
+// T256 B32 D256 H512).  Several launches, whose dW_hh would otherwise be less accurate than
+// the per-step path's, and smaller KQ, where they cost nothing measurable, take WS = 2.
+int wgrad_form(int kq, int launches) { return !split_products_mode() ? 0 : kq == 128 && launches == 1 ? 1 : 2; }
+
+template <int KQ, int WS>
 int bwd_resident_ws(int xt, int* occ) {
   int o = 0;
   switch (xt) {
     case -1:
-      HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, rec_bwd_persistent<KQ, -1, true>, 256,
+      HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, rec_bwd_persistent<KQ, -1, 2>, 256,
                                                            bwd_lds_bytes(-1, true)));
       break;
     case 0:
@@ -2106,8 +2116,9 @@ int bwd_resident_ws(int xt, int* occ) {
   return HSL_OK;
 }
 template <int KQ>
-int bwd_resident(int xt, bool ws, int* occ) {
-  return ws ? bwd_resident_ws<KQ, true>(xt, occ) : bwd_resident_ws<KQ, false>(xt, occ);
+int bwd_resident(int xt, int ws, int* occ) {
+  if (KQ == 128 && ws == 1) return bwd_resident_ws<KQ, (KQ == 128 ? 1 : 2)>(xt, occ);
+  return ws ? bwd_resident_ws<KQ, 2>(xt, occ) : bwd_resident_ws<KQ, 0>(xt, occ);
 }
 
 // Launches a batch may be split into before the per-step path takes over.  One launch costs
@@ -2140,7 +2151,7 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
   // x rows with 16-byte loads
   if (!bwd && fused_xproj_enabled()) p.XP = D > 0 && D <= 256 && D % 4 == 0;
   p.XS = kXprojSplit && split_products_mode();
-  p.WS = split_products_mode() != 0;
+  p.WS = wgrad_form(kq, 1);
   int occ = 0;
   for (;;) {
     if (bwd) {
@@ -2171,6 +2182,7 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
       p.NGX = (p.gpl + di.num_xcds - 1) / di.num_xcds * di.num_xcds;
       p.grid = p.NGX * p.NW;
       p.ok = p.launches <= (mode == 2 ? 1 : kMaxGroupLaunches);
+      p.WS = wgrad_form(kq, p.launches);
     }
     if (p.ok || fit > 0 || (p.XT < 0 && !p.XP)) break;
     p.XT = -1;  // retry without the weight-gradient / projection waves
@@ -2180,12 +2192,13 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
   return HSL_OK;
 }
 
-// The W_hh-resident kernels for large H (rec_wide.h, rec_wide_fwd.h, rec_wide_bwd32.h): H = 32 U
-// with U = 64 (2048) or 32 (1024), B <= 32, eight XCDs and all 256 workgroups resident at
-// once (one per CU).
+// The W_hh-resident kernels for large H (rec_wide.h, rec_wide_fwd.h, rec_wide_bwd32.h): widths
+// 32 U with U = 32 (512 < H <= 1024) or 64 (1024 < H <= 2048), eight XCDs and all 256
+// workgroups resident at once (one per CU); one launch per 32 batch rows.
 struct WidePlan {
   bool ok = false;
   int U = 0;
+  int rows = 0;  // batch rows per launch
 };
 
 // dynamic LDS of the wide kernels, padded so that one workgroup fits per CU: the forward's
@@ -2209,30 +2222,54 @@ size_t wide_fwd_floats(int U) {
 size_t wide_bwd_bfloats(int U) { return (size_t)kWideHSlots * kWideXcds * (16 * U) * 32; }
 size_t wide_bwd_floats(int U) { return wide_bwd_bfloats(U) + (size_t)kWidePSlots * kWideWgs * (8 * 32 * (U / 8)); }
 
+template <int U, bool PAD>
+const void* wide_kernel(bool bwd) {
+  if (!bwd) return (const void*)rec_fwd_wide<U, PAD>;
+  return U == 32 ? (const void*)rec_bwd_wide1<32, PAD> : (const void*)rec_bwd_wide<64, PAD>;
+}
 template <int U>
-int wide_occupancy(bool bwd, int* occ) {
-  if (bwd)
-    HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        occ, U == 32 ? (const void*)rec_bwd_wide1<32> : (const void*)rec_bwd_wide<64>, 256, wide_bwd_lds<U>()));
-  else
-    HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, rec_fwd_wide<U>, 256, wide_fwd_lds<U>()));
+int wide_occupancy(bool bwd, bool pad, int* occ) {
+  HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, pad ? wide_kernel<U, true>(bwd) : wide_kernel<U, false>(bwd),
+                                                       256, bwd ? wide_bwd_lds<U>() : wide_fwd_lds<U>()));
   return HSL_OK;
+}
+
+// The width of the wide kernels that hold a hidden size (units per k block / 4), 0 = none.
+int wide_u(int H) { return H > 512 && H <= 1024 ? 32 : H > 1024 && H <= 2048 ? 64 : 0; }
+
+// Launches (of 32 batch rows) up to which the wide kernels beat the per-step path.  A launch
+// costs the width's time whatever H and the rows are; the per-step path's cost grows slowly
+// with B, and is higher where H is no multiple of 4 (4-byte loads).  us per step (forward,
+// backward with its products) at T = 32, D = 256, wide against per step:
+//   B = 32: H = 520 6.9, 10.5 / 10.1, 15.2;  H = 1024 6.7, 10.5 / 11.5, 16.6;
+//           H = 1100 13.1, 25.6 / 14.4, 26.3;  H = 2048 13.1, 23.3 / 20.0, 31.6
+//   B = 64: H = 520 12.9, 19.1 / 12.2, 16.6;  H = 650 13.4, 21.1 / 19.9, 23.5;
+//           H = 1024 13.5, 20.0 / 11.9, 20.8;  H = 1100 28.0, 49.0 / 25.8, 39.0;
+//           H = 1500 28.3, 62.1 / 31.0, 66.2;  H = 2048 25.2, 43.7 / 30.6, 45.3
+//   B = 128: H = 1500 53.5, 116 / 42.9, 113;  H = 2048 50.7, 89.5 / 64.0, 97.7
+int wide_launches(int H) {
+  if (H <= 1024) return H % 4 ? 2 : 1;
+  return H < 1408 ? 1 : H < 1792 ? 2 : 4;
 }
 
 int plan_wide(int B, int H, bool bwd, WidePlan* pl) {
   *pl = WidePlan{};
-  if (recurrent_path_mode() == 1 || B < 1 || B > 32 || (H != 2048 && H != 1024)) return HSL_OK;
+  const int mode = recurrent_path_mode();
+  const int U = wide_u(H);
+  if (mode == 1 || B < 1 || U == 0) return HSL_OK;
+  const int launches = (B + 31) / 32;
+  if (launches > wide_launches(H) || (mode == 2 && (launches > 1 || H != 32 * U))) return HSL_OK;
   DeviceInfo di;
   HSL_CHECK(device_info(&di));
   if (di.num_xcds != kWideXcds || di.num_cus < kWideWgs) return HSL_OK;
-  const int U = H / 32;
   int occ = 0;
   if (U == 64)
-    HSL_CHECK(wide_occupancy<64>(bwd, &occ));
+    HSL_CHECK(wide_occupancy<64>(bwd, H != 32 * U, &occ));
   else
-    HSL_CHECK(wide_occupancy<32>(bwd, &occ));
+    HSL_CHECK(wide_occupancy<32>(bwd, H != 32 * U, &occ));
   pl->ok = occ >= 1 && (long)occ * di.num_cus >= kWideWgs;
   pl->U = U;
+  pl->rows = (B + launches - 1) / launches;
   return HSL_OK;
 }
 
@@ -2279,10 +2316,11 @@ int fill_words(unsigned long long* p, size_t n, unsigned long long v, hipStream_
 }
 
 // Before a persistent launch: error flag cleared, hand-off slots empty (every 4-byte
-// word kEmpty), placement words cleared, in one launch.
+// word kEmpty), placement words cleared, in one launch.  A later launch of the same call
+// that reuses the slots passes no error flag, so that it keeps what the earlier ones raised.
 int prepare_persistent(int* err, float* slots, size_t slot_floats, unsigned long long* hello, size_t hwords,
                        hipStream_t s) {
-  const size_t n1 = 32, n2 = (slot_floats + 1) / 2;
+  const size_t n1 = err ? 32 : 0, n2 = (slot_floats + 1) / 2;
   hipLaunchKernelGGL(fill3_u64_kernel, dim3(grid_for(n1 + (n2 + 1) / 2 + hwords)), dim3(256), 0, s,
                      reinterpret_cast<unsigned long long*>(err), n1, 0ull,
                      reinterpret_cast<unsigned long long*>(slots), n2, kEmpty2, hello, hwords, 0ull);
@@ -2333,9 +2371,9 @@ size_t carve_fwd(void* ws, size_t cap, int T, int B, int H, FwdNeeds nd, FwdWs* 
     o->hello = c.take<unsigned long long>(o->hwords);
   }
   if (nd.gih) o->gih = c.take<float>((size_t)T * B * 4 * H);
-  if (nd.wide && (H == 2048 || H == 1024)) {
-    o->whfloats = wide_fwd_hfloats(H / 32);
-    o->wfloats = wide_fwd_floats(H / 32);
+  if (const int U = wide_u(H); nd.wide && U) {
+    o->whfloats = wide_fwd_hfloats(U);
+    o->wfloats = wide_fwd_floats(U);
     o->wbuf = c.take<float>(o->wfloats);
     o->whello = c.take<unsigned long long>(kWideWgs);
   }
@@ -2439,8 +2477,8 @@ size_t carve_bwd(void* ws, size_t cap, int T, int B, int D, int H, BwdNeeds nd, 
     o->pbuf = c.take<float>(o->pfloats);
     o->hello = c.take<unsigned long long>(o->hwords);
   }
-  if (nd.wide && (H == 2048 || H == 1024)) {
-    o->wfloats = wide_bwd_floats(H / 32);
+  if (const int U = wide_u(H); nd.wide && U) {
+    o->wfloats = wide_bwd_floats(U);
     o->wbuf = c.take<float>(o->wfloats);
     o->whello = c.take<unsigned long long>(kWideWgs);
   }
@@ -2460,11 +2498,11 @@ void launch_fwd_persistent(const PFwdArgs& a, int grid, int xp, hipStream_t s) {
     default: hipLaunchKernelGGL((rec_fwd_persistent<KQ, 2>), dim3(grid), dim3(512), kFwdLdsBytes, s, a); break;
   }
 }
-template <int KQ, bool WS>
+template <int KQ, int WS>
 void launch_bwd_persistent_ws(const PBwdArgs& a, int grid, int xt, hipStream_t s) {
   switch (xt) {
     case -1:
-      hipLaunchKernelGGL((rec_bwd_persistent<KQ, -1, true>), dim3(grid), dim3(256), bwd_lds_bytes(-1, true), s, a);
+      hipLaunchKernelGGL((rec_bwd_persistent<KQ, -1, 2>), dim3(grid), dim3(256), bwd_lds_bytes(-1, true), s, a);
       break;
     case 0:
       hipLaunchKernelGGL((rec_bwd_persistent<KQ, 0, WS>), dim3(grid), dim3(512), bwd_lds_bytes(0, WS), s, a);
@@ -2475,11 +2513,13 @@ void launch_bwd_persistent_ws(const PBwdArgs& a, int grid, int xt, hipStream_t s
   }
 }
 template <int KQ>
-void launch_bwd_persistent(const PBwdArgs& a, int grid, int xt, bool ws, hipStream_t s) {
-  if (ws)
-    launch_bwd_persistent_ws<KQ, true>(a, grid, xt, s);
+void launch_bwd_persistent(const PBwdArgs& a, int grid, int xt, int ws, hipStream_t s) {
+  if (KQ == 128 && ws == 1)
+    launch_bwd_persistent_ws<KQ, (KQ == 128 ? 1 : 2)>(a, grid, xt, s);
+  else if (ws)
+    launch_bwd_persistent_ws<KQ, 2>(a, grid, xt, s);
   else
-    launch_bwd_persistent_ws<KQ, false>(a, grid, xt, s);
+    launch_bwd_persistent_ws<KQ, 0>(a, grid, xt, s);
 }
 
 }  // namespace
@@ -2623,14 +2663,19 @@ int hsl_rec_fwd(const float* x, const float* h0, const float* c0, const float* w
     return HSL_OK;
   }
   if (wp.ok) {
-    WFwdArgs wa{w.gih, w_hh, b_hh, a, h0, c0, h_save, c_save, gact, tanh_c, w.wbuf, w.wbuf + w.whfloats, w.whello,
-                w.err, T, B, H, exchange_scope_mode(), spin_timeout_ticks()};
     const int slot = timing_begin(kTimeRecFwd, s);
-    if (wp.U == 64)
-      hipLaunchKernelGGL(rec_fwd_wide<64>, dim3(kWideWgs), dim3(256), wide_fwd_lds<64>(), s, wa);
-    else
-      hipLaunchKernelGGL(rec_fwd_wide<32>, dim3(kWideWgs), dim3(256), wide_fwd_lds<32>(), s, wa);
-    HSL_HIP(hipGetLastError());
+    for (int b0 = 0; b0 < B; b0 += wp.rows) {
+      if (b0 > 0) HSL_CHECK(prepare_persistent(nullptr, w.wbuf, w.wfloats, w.whello, kWideWgs, s));
+      const size_t o = (size_t)b0 * H;
+      WFwdArgs wa{w.gih + 4 * o, w_hh, b_hh, a, h0 ? h0 + o : nullptr, c0 ? c0 + o : nullptr, h_save + o, c_save + o,
+                  gact + 4 * o, tanh_c + o, w.wbuf, w.wbuf + w.whfloats, w.whello, w.err, T, B, H,
+                  std::min(wp.rows, B - b0), exchange_scope_mode(), spin_timeout_ticks()};
+      const auto kernel = wp.U == 64 ? (H == 2048 ? rec_fwd_wide<64, false> : rec_fwd_wide<64, true>)
+                                     : (H == 1024 ? rec_fwd_wide<32, false> : rec_fwd_wide<32, true>);
+      hipLaunchKernelGGL(kernel, dim3(kWideWgs), dim3(256), wp.U == 64 ? wide_fwd_lds<64>() : wide_fwd_lds<32>(), s,
+                         wa);
+      HSL_HIP(hipGetLastError());
+    }
     timing_end(slot, s);
     note_recurrent_path(3);
     return HSL_OK;
@@ -2795,15 +2840,20 @@ int hsl_rec_bwd(const float* dout, const float* dh_n, const float* dc_n, const f
     note_backward_fused(fused_ih ? 2 : fused ? 1 : 0);
   } else if (wp.ok) {
     note_backward_fused(0);
-    WBwdArgs wa{dout, dh_n, dc_n, c_save, gact, tanh_c, w_hh, a, w.dgates, w.db_part, dh0, dc0, w.wbuf,
-                w.wbuf + wide_bwd_bfloats(wp.U), w.whello, w.err, T, B, H,
-                exchange_scope_mode(), spin_timeout_ticks()};
     const int slot = timing_begin(kTimeRecBwd, s);
-    if (wp.U == 64)
-      hipLaunchKernelGGL(rec_bwd_wide<64>, dim3(kWideWgs), dim3(256), wide_bwd_lds<64>(), s, wa);
-    else
-      hipLaunchKernelGGL(rec_bwd_wide1<32>, dim3(kWideWgs), dim3(256), wide_bwd_lds<32>(), s, wa);
-    HSL_HIP(hipGetLastError());
+    for (int b0 = 0; b0 < B; b0 += wp.rows) {
+      if (b0 > 0) HSL_CHECK(prepare_persistent(nullptr, w.wbuf, w.wfloats, w.whello, kWideWgs, s));
+      const size_t o = (size_t)b0 * H;
+      auto at = [o](auto* ptr) { return ptr ? ptr + o : nullptr; };
+      WBwdArgs wa{dout + o, at(dh_n), at(dc_n), c_save + o, gact + 4 * o, tanh_c + o, w_hh, a, w.dgates + 4 * o,
+                  w.db_part + 4 * o, at(dh0), at(dc0), w.wbuf, w.wbuf + wide_bwd_bfloats(wp.U), w.whello, w.err,
+                  T, B, H, std::min(wp.rows, B - b0), exchange_scope_mode(), spin_timeout_ticks()};
+      const auto kernel = wp.U == 64 ? (H == 2048 ? rec_bwd_wide<64, false> : rec_bwd_wide<64, true>)
+                                     : (H == 1024 ? rec_bwd_wide1<32, false> : rec_bwd_wide1<32, true>);
+      hipLaunchKernelGGL(kernel, dim3(kWideWgs), dim3(256), wp.U == 64 ? wide_bwd_lds<64>() : wide_bwd_lds<32>(), s,
+                         wa);
+      HSL_HIP(hipGetLastError());
+    }
     timing_end(slot, s);
     note_recurrent_path(3);
   } else {

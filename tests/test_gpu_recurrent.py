@@ -230,6 +230,19 @@ def test_wide_short_sequences(dev, T, B, H):
     assert prlstm_amd.last_recurrent_path() == 3
 
 
+@pytest.mark.parametrize("T,B,H", [(7, 5, 513), (6, 20, 650), (9, 32, 771), (5, 18, 1023),    # width 1024
+                                   (6, 3, 1025), (5, 32, 1500), (4, 17, 2047),               # width 2048
+                                   (6, 33, 650), (3, 50, 1500), (2, 70, 1800)])              # two and three launches
+def test_wide_kernels_padded_width_and_batch_launches(dev, T, B, H):
+    """Hidden sizes between the wide kernels' own widths run on the next width, whose units past
+    H keep every hand-off's order but read and store nothing (H a multiple of 4 or not: 16- or
+    4-byte loads of W_hh), and batches beyond 32 rows as launches of at most 32 rows."""
+    for scope in (0, 1) if H in (650, 1500) else (0,):
+        prlstm_amd.set_exchange_scope(scope)
+        check(T, B, 24, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=True, fwd_path=3)
+        assert prlstm_amd.last_recurrent_path() == 3
+
+
 def test_sgd_training_step(dev):
     """test_cpp.py:110-147: one SGD step (MSE loss), updated parameters agree."""
     T, B, D, H, lr = 12, 4, 8, 12, 1e-2
