@@ -254,6 +254,34 @@ __global__ __launch_bounds__(1024) void bias_da_finalize_kernel(const double* __
   if (threadIdx.x == 0 && da) da[g] = (float)red[0];
 }
 
+// db[n] = sum_r part[r][n] over `rows` rows of `cols` fp64 partials, without the da term:
+// 64 columns per workgroup, wave w adds rows w, w + 16, ... and the 16 sums are added in wave
+// order.  The parallel backward's rows are its batch rows times the scan's segments of T;
+// one workgroup per gate (bias_da_finalize_kernel) would add them on four CUs.
+__global__ __launch_bounds__(1024) void colsum_parts_kernel(const double* __restrict__ part, int rows, int cols,
+                                                            float* __restrict__ db) {
+  __shared__ double red[16][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, n = blockIdx.x * 64 + lane;
+  const double* const p = part + min(n, cols - 1);
+  double acc = 0.0;
+  constexpr int kBatch = 4;  // rows in flight
+  for (int r0 = w; r0 < rows; r0 += 16 * kBatch) {
+    double v[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) v[i] = r0 + 16 * i < rows ? p[(size_t)(r0 + 16 * i) * cols] : 0.0;
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) acc += v[i];
+  }
+  red[w][lane] = acc;
+  __syncthreads();
+  if (w == 0 && n < cols) {
+    double s = 0.0;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) s += red[u][lane];
+    db[n] = (float)s;
+  }
+}
+
 // ---------------------------------------------------------------------------------
 // per-step path: fused epilogues of the step GEMMs
 // ---------------------------------------------------------------------------------
@@ -2531,6 +2559,11 @@ int bias_grads_from_parts(const double* db_part, int B, const double* rowdot, co
                           float* db_ih, float* db_hh, float* da, int H, hipStream_t s, const double* dotp,
                           int dot_parts) {
   if (H == 0) return HSL_OK;
+  if (!da && !db_hh && db_ih) {
+    hipLaunchKernelGGL(colsum_parts_kernel, dim3((4 * H + 63) / 64), dim3(1024), 0, s, db_part, B, 4 * H, db_ih);
+    HSL_HIP(hipGetLastError());
+    return HSL_OK;
+  }
   hipLaunchKernelGGL(bias_da_finalize_kernel, dim3(4), dim3(1024), 0, s, db_part, B, rowdot, b_hh, a, db_ih, db_hh,
                      da, H, dotp, dot_parts);
   HSL_HIP(hipGetLastError());

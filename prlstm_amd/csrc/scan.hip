@@ -17,7 +17,8 @@
 //
 // Layout: gates [T,B,4H] (the GEMM output, never transposed), out [T,B,H].  One
 // workgroup owns 64 consecutive channels (b,j) = one wave-width, so every load and
-// store is a 256-byte row segment, and walks all of T in chunks of NW*L steps: each
+// store is a 256-byte row segment, and walks all of T (or, with few channels, one of the
+// segments that T is cut into, see scan_fwd_map_kernel) in chunks of NW*L steps: each
 // of the NW waves takes L consecutive steps, composes them into one map, the maps
 // are combined through LDS, and each wave re-runs its steps from its carry-in.  The
 // next chunk's loads are issued before the current chunk is processed.  Every [T,...]
@@ -90,7 +91,7 @@ constexpr int kCkSteps = 8;  // steps per checkpoint row of c (one wave's group 
 template <int NW, int L, int OF>
 __global__ __launch_bounds__(NW * 64) void scan_fwd_kernel(const float* __restrict__ gates, const float* __restrict__ c0,
                                                           float eps, void* __restrict__ out, float* __restrict__ cck,
-                                                          int T, int B, int H) {
+                                                          int T, int B, int H, int seg) {
   static_assert(L == kCkSteps, "checkpoint rows are one per L-step group");
   __shared__ float2 sAV[NW][64];  // each wave's composed map (A, V) of the chunk
   __shared__ float sC[64];
@@ -109,10 +110,12 @@ __global__ __launch_bounds__(NW * 64) void scan_fwd_kernel(const float* __restri
   const unsigned orow_o = (unsigned)ostride * OB, ov_o = ok ? (unsigned)ch * OB : kOffNone;
   char* const outb = static_cast<char*>(out);
   const int hb = 4 * H;  // bytes between gate planes
-  if (w == 0) sC[lane] = ok ? fmaxf(c0 ? c0[ch] : 0.f, eps) : 0.f;
-
   constexpr int CH = NW * L;
-  const int nchunks = (T + CH - 1) / CH, nfull = T / CH;
+  // this workgroup's chunks k0 .. nchunks-1; a segment past the first starts from the state
+  // that scan_fwd_carry_kernel left in its first checkpoint row
+  const int k0 = blockIdx.y * seg;
+  const int nchunks = min(k0 + seg, (T + CH - 1) / CH), nfull = min(nchunks, T / CH);
+  if (w == 0) sC[lane] = !ok ? 0.f : k0 > 0 ? cck[(size_t)k0 * NW * ostride + ch] : fmaxf(c0 ? c0[ch] : 0.f, eps);
   const int nck = (T + L - 1) / L;  // the c_n row
   // the step loads: rows past T have size 0 (they read 0)
   auto load = [&](int chunk, float(&r)[4][L]) {
@@ -179,8 +182,8 @@ __global__ __launch_bounds__(NW * 64) void scan_fwd_kernel(const float* __restri
   };
   // chunks alternate between two register sets, so no copies between them
   float ra[4][L], rb[4][L];
-  if (nchunks > 0) load(0, ra);
-  int k = 0;
+  if (nchunks > k0) load(k0, ra);
+  int k = k0;
   for (; k + 1 < nfull; k += 2) {
     chunk(std::false_type{}, k, ra, rb);
     chunk(std::false_type{}, k + 1, rb, ra);
@@ -197,7 +200,7 @@ template <int NW, int L, int DF>
 __global__ __launch_bounds__(NW * 64) void scan_bwd_kernel(
     const float* __restrict__ gates, const float* __restrict__ c0, const float* __restrict__ cck,
     const void* __restrict__ dout, const float* __restrict__ dh_n, const float* __restrict__ dc_n, float eps,
-    float* __restrict__ dgates, double* __restrict__ db_part, float* __restrict__ dc0, int T, int B, int H) {
+    float* __restrict__ dgates, double* __restrict__ db_part, float* __restrict__ dc0, int T, int B, int H, int seg) {
   static_assert(L == kCkSteps, "a wave's steps are one checkpoint group");
   __shared__ float2 sAV[NW][64];  // each wave's composed reverse map (A, V) of the chunk
   __shared__ float sG[64];
@@ -220,10 +223,12 @@ __global__ __launch_bounds__(NW * 64) void scan_bwd_kernel(
   const float c0v = (ok && c0) ? c0[ch] : 0.f;
   const bool c0_pass = ok && c0v >= eps;
   const float dhn = (ok && dh_n) ? dh_n[ch] : 0.f, dcn = (ok && dc_n) ? dc_n[ch] : 0.f;
-  if (w == 0) sG[lane] = 0.f;
-
   constexpr int CH = NW * L;
-  const int nchunks = (T + CH - 1) / CH;
+  // this workgroup's chunks k0 .. nchunks-1; a segment before the last starts from the G that
+  // scan_bwd_carry_kernel left in the g-gate words of its first dgates row
+  const int k0 = blockIdx.y * seg, allchunks = (T + CH - 1) / CH;
+  const int nchunks = min(k0 + seg, allchunks);
+  if (w == 0) sG[lane] = ok && nchunks < allchunks ? dgates[(size_t)k0 * CH * gstride + (size_t)b * 4 * H + 2 * H + j] : 0.f;
   // per step: zi zf zg zo dout; plus zf at we+1 (fnext) and the group's checkpoint row, the
   // c carried into its first step (cin); rows past T read 0
   auto load = [&](int chunk, float(&r)[5][L], float& fnext, float& cin) {
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(NW * 64) void scan_bwd_kernel(
   auto chunk = [&](auto last, int k, float(&cur)[5][L], float cur_fn, float cur_cin, float(&nxt)[5][L],
                    float& nxt_fn, float& nxt_cin) {
     constexpr bool LAST = decltype(last)::value;
-    if (k > 0) load(k - 1, nxt, nxt_fn, nxt_cin);
+    if (k > k0) load(k - 1, nxt, nxt_fn, nxt_cin);
     const int ws = k * CH + w * L;
     // sigma(z_f), sigma(z_o), c and tanh(c) of each step, computed once and used by both
     // passes; c_t is recomputed from the carry-in by the forward's own operations, so it
@@ -344,18 +349,18 @@ __global__ __launch_bounds__(NW * 64) void scan_bwd_kernel(
   // chunks alternate between two register sets, so no copies between them
   float ra[5][L], rb[5][L];
   float fa = 0.f, pa = 0.f, fb = 0.f, pb = 0.f;
-  if (nchunks > 0) {
+  if (nchunks > k0) {
     load(nchunks - 1, ra, fa, pa);
     chunk(std::true_type{}, nchunks - 1, ra, fa, pa, rb, fb, pb);
   }
   int k = nchunks - 2;
-  for (; k >= 1; k -= 2) {
+  for (; k >= k0 + 1; k -= 2) {
     chunk(std::false_type{}, k, rb, fb, pb, ra, fa, pa);
     chunk(std::false_type{}, k - 1, ra, fa, pa, rb, fb, pb);
   }
-  if (k == 0) chunk(std::false_type{}, 0, rb, fb, pb, ra, fa, pa);
+  if (k == k0) chunk(std::false_type{}, k0, rb, fb, pb, ra, fa, pa);
   // dc0 = G_0 f~_0 where the clamp of c0 passes gradient
-  if (w == 0 && ok && dc0) dc0[ch] = (c0_pass && T > 0) ? g_first * f_first : 0.f;
+  if (w == 0 && ok && dc0 && k0 == 0) dc0[ch] = (c0_pass && T > 0) ? g_first * f_first : 0.f;
   if (db_part) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) sdb[w][g][lane] = dbacc[g];
@@ -365,10 +370,212 @@ __global__ __launch_bounds__(NW * 64) void scan_bwd_kernel(
       for (int g = 0; g < 4; ++g) {
         double s = 0.0;
         for (int u = 0; u < NW; ++u) s += sdb[u][g][lane];
-        db_part[(size_t)b * 4 * H + g * H + j] = s;
+        db_part[((size_t)blockIdx.y * B + b) * 4 * H + g * H + j] = s;
       }
     }
   }
+}
+
+// ---- few channels: T split into segments of whole chunks --------------------------------
+// A workgroup per 64 channels leaves the chip idle when B*H is small (T16384 B2 H256: 8
+// workgroups, 600 us forward and 965 us backward for 0.48 GB).  Both recurrences are affine,
+// so T is then cut into segments that run as workgroups of their own:
+//   1. scan_*_map_kernel composes each segment's steps into one affine map (A, V);
+//   2. scan_*_carry_kernel, one thread per channel, carries the state across the segments;
+//   3. the scan kernels run each segment from its carried state.
+// Maps and carried states live in rows of the call's own outputs that pass 3 overwrites, so
+// no workspace is needed: forward in c_ck rows of the segment (state in its first, which is
+// that row's value anyway, A and V in the next two); backward in the segment's first dgates
+// row (A, V and the carried G in the words of gates i, f and g).  Pass 1 reads 12 of the
+// forward's 20 bytes per element and 20 of the backward's 36 once more.
+constexpr int kMapWaves = 16;
+
+// Forward map of segment blockIdx.y (never the last one, so every step is below T): wave w
+// composes the w-th part of its `steps` steps in groups of 8.
+__global__ __launch_bounds__(kMapWaves * 64) void scan_fwd_map_kernel(const float* __restrict__ gates, float eps,
+                                                                     float* __restrict__ cck, int steps, int B, int H) {
+  __shared__ float2 sAV[kMapWaves][64];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int C = B * H, ch = blockIdx.x * 64 + lane;
+  const bool ok = ch < C;
+  const int b = ok ? ch / H : 0, j = ok ? ch % H : 0;
+  const size_t gstride = (size_t)B * 4 * H;
+  const unsigned grow = (unsigned)(gstride * 4), gv = ok ? (unsigned)(b * 4 * H + j) * 4u : kOffNone;
+  const int hb = 4 * H, part = steps / kMapWaves;  // a multiple of 8
+  const int t0 = blockIdx.y * steps + w * part;
+  float A = 1.f, V = 0.f;
+  for (int g0 = 0; g0 < part; g0 += kCkSteps) {
+    float z[3][kCkSteps];
+#pragma unroll
+    for (int s = 0; s < kCkSteps; ++s) {
+      const auto rs = row_rsrc(gates + (size_t)(t0 + g0 + s) * gstride, grow);
+#pragma unroll
+      for (int g = 0; g < 3; ++g) z[g][s] = row_load<0>(rs, gv, g * hb);  // read again by pass 3
+    }
+#pragma unroll
+    for (int s = 0; s < kCkSteps; ++s) {
+      const float f = fmaxf(sigmoid_f(z[1][s]), eps);
+      const float bb = fmaxf(sigmoid_prod_f(z[0][s], z[2][s]), eps);
+      A = f * A;
+      V = f * V + bb;
+    }
+  }
+  sAV[w][lane] = float2{A, V};
+  __syncthreads();
+  if (w == 0 && ok) {
+    A = 1.f;
+    V = 0.f;
+#pragma unroll
+    for (int u = 0; u < kMapWaves; ++u) {
+      const float2 m = sAV[u][lane];
+      A = m.x * A;
+      V = m.x * V + m.y;
+    }
+    float* const row = cck + ((size_t)blockIdx.y * steps / kCkSteps + 1) * C + ch;
+    row[0] = A;
+    row[C] = V;
+  }
+}
+
+// c into every segment past the first: row p * steps / 8 of c_ck.
+__global__ __launch_bounds__(64) void scan_fwd_carry_kernel(const float* __restrict__ c0, float eps, float* cck,
+                                                            int steps, int nseg, int C) {
+  const int ch = blockIdx.x * 64 + threadIdx.x;
+  if (ch >= C) return;
+  const size_t seg = (size_t)steps / kCkSteps * C;
+  constexpr int kBatch = 8;  // maps in flight
+  float c = fmaxf(c0 ? c0[ch] : 0.f, eps);
+  for (int p0 = 0; p0 + 1 < nseg; p0 += kBatch) {
+    float A[kBatch], V[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const float* const row = cck + min(p0 + i, nseg - 2) * seg + C + ch;
+      A[i] = row[0];
+      V[i] = row[C];
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+      if (p0 + i + 1 < nseg) {
+        c = A[i] * c + V[i];
+        cck[(p0 + i + 1) * seg + ch] = c;
+      }
+  }
+}
+
+// Reverse map of segment blockIdx.y + 1 (never the first): wave w composes the w-th part of
+// its `steps` steps, from the last group of 8 to the first, each group from its checkpoint row.
+template <int DF>
+__global__ __launch_bounds__(kMapWaves * 64) void scan_bwd_map_kernel(
+    const float* __restrict__ gates, const float* __restrict__ cck, const void* __restrict__ dout,
+    const float* __restrict__ dh_n, const float* __restrict__ dc_n, float eps, float* __restrict__ dgates, int steps,
+    int T, int B, int H) {
+  __shared__ float2 sAV[kMapWaves][64];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int C = B * H, ch = blockIdx.x * 64 + lane;
+  const bool ok = ch < C;
+  const int b = ok ? ch / H : 0, j = ok ? ch % H : 0;
+  const size_t gstride = (size_t)B * 4 * H;
+  const unsigned grow = (unsigned)(gstride * 4), orow = 4u * C, drow = fmt_bytes<DF>() * C;
+  const unsigned gv = ok ? (unsigned)(b * 4 * H + j) * 4u : kOffNone, ov = ok ? (unsigned)ch * 4u : kOffNone;
+  const unsigned dv = ok ? (unsigned)ch * fmt_bytes<DF>() : kOffNone;
+  const char* const doutb = static_cast<const char*>(dout);
+  const float dhn = (ok && dh_n) ? dh_n[ch] : 0.f, dcn = (ok && dc_n) ? dc_n[ch] : 0.f;
+  const int hb = 4 * H, part = steps / kMapWaves;
+  const int ts = ((int)blockIdx.y + 1) * steps, t0 = ts + w * part;
+  float A = 1.f, V = 0.f;
+  for (int g0 = part - kCkSteps; g0 >= 0; g0 -= kCkSteps) {
+    const int ws = t0 + g0;
+    if (ws >= T) continue;
+    float z[4][kCkSteps], d[kCkSteps];
+#pragma unroll
+    for (int s = 0; s < kCkSteps; ++s) {  // rows past T have size 0 (they read 0)
+      const auto rg = row_rsrc(gates + (size_t)(ws + s) * gstride, ws + s < T ? grow : 0u);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) z[g][s] = row_load<0>(rg, gv, g * hb);
+      d[s] = in_load<DF>(row_rsrc(reinterpret_cast<const float*>(doutb + (size_t)(ws + s) * drow), ws + s < T ? drow : 0u),
+                         dv, 0);
+    }
+    const int tn = ws + kCkSteps;
+    const float zn = row_load<0>(row_rsrc(gates + (size_t)tn * gstride, tn < T ? grow : 0u), gv, hb);
+    float c = row_load<0>(row_rsrc(cck + (size_t)(ws / kCkSteps) * C, orow), ov, 0);
+    float fg[kCkSteps], ev[kCkSteps];
+#pragma unroll
+    for (int s = 0; s < kCkSteps; ++s) {
+      const int t = ws + s;
+      fg[s] = fmaxf(sigmoid_f(z[1][s]), eps);
+      c = __builtin_fmaf(fg[s], c, fmaxf(sigmoid_prod_f(z[0][s], z[2][s]), eps));
+      const float tc = tanh_pos_f(c);
+      const float e = (t == T - 1 ? d[s] + dhn : d[s]) * sigmoid_f(z[3][s]) * (1.0f - tc * tc);
+      ev[s] = t == T - 1 ? e + dcn : e;
+    }
+    const float fn = fmaxf(sigmoid_f(zn), eps);
+#pragma unroll
+    for (int s = kCkSteps - 1; s >= 0; --s) {
+      const int t = ws + s;
+      if (t < T) {
+        const float f = t + 1 < T ? (s + 1 < kCkSteps ? fg[s + 1 < kCkSteps ? s + 1 : 0] : fn) : 0.f;
+        V = ev[s] + f * V;
+        A = f * A;
+      }
+    }
+  }
+  sAV[w][lane] = float2{A, V};
+  __syncthreads();
+  if (w == 0 && ok) {
+    A = 1.f;
+    V = 0.f;
+#pragma unroll
+    for (int u = kMapWaves - 1; u >= 0; --u) {
+      const float2 m = sAV[u][lane];
+      A = m.x * A;
+      V = m.x * V + m.y;
+    }
+    float* const row = dgates + (size_t)ts * gstride + (size_t)b * 4 * H + j;
+    row[0] = A;
+    row[H] = V;
+  }
+}
+
+// G into every segment before the last: the g-gate words of its first dgates row.
+__global__ __launch_bounds__(64) void scan_bwd_carry_kernel(float* dgates, int steps, int nseg, int B, int H) {
+  const int ch = blockIdx.x * 64 + threadIdx.x;
+  if (ch >= B * H) return;
+  const size_t seg = (size_t)steps * B * 4 * H;
+  float* const col = dgates + (size_t)(ch / H) * 4 * H + ch % H;
+  constexpr int kBatch = 8;
+  float G = 0.f;
+  for (int p0 = nseg - 1; p0 > 0; p0 -= kBatch) {
+    float A[kBatch], V[kBatch];
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i) {
+      const float* const row = col + max(p0 - i, 1) * seg;
+      A[i] = row[0];
+      V[i] = row[H];
+    }
+#pragma unroll
+    for (int i = 0; i < kBatch; ++i)
+      if (p0 - i > 0) {
+        G = A[i] * G + V[i];
+        col[(p0 - i - 1) * seg + 2 * H] = G;
+      }
+  }
+}
+
+// Chunks (of `chunk` steps) per segment: all of them unless 64-channel workgroups leave many
+// of the chip's CUs without one; then about one workgroup per CU.  us (forward, backward) of
+// one segment against segments for 256 workgroups (128 and 512 are no better), H = 512:
+//   T = 16384, 8 groups of 64 channels (H = 256): 602, 978 / 74, 122
+//   T = 4096, 32 groups: 157, 251 / 57, 92;      T = 2048, 64 groups: 85, 133 / 55, 85
+//   T = 2048, 96 groups: 89, 144 / 80, 134;      T = 2048, 128 groups: 92, 155 / 90, 155
+//   T = 512, 16 groups: 21, 38 / 15, 26;         T = 300, 5 groups (H = 100): 22, 27 / 17, 25
+//   T = 256, 16 groups (H = 256): 12.5, 22.1 / 14.6, 23.1 -> at least `least` chunks
+int scan_seg_chunks(int T, long C, int chunk, int least) {
+  const int groups = (int)((C + 63) / 64), nchunks = (T + chunk - 1) / chunk;
+  if (groups > 96 || nchunks < least) return nchunks;
+  const int nseg = std::min(nchunks, 256 / groups);
+  return nseg < 2 ? nchunks : (nchunks + nseg - 1) / nseg;
 }
 
 // one time step of gates (16 B H bytes) is addressed as a buffer of < 2^31 bytes
@@ -380,24 +587,41 @@ int scan_fwd(const float* gates, const float* c0, float eps, void* out, float* c
   const int C = B * H;
   if (C == 0 || T == 0) return HSL_OK;
   const int slot = timing_begin(kTimeScanFwd, s);
-  const dim3 grid((C + 63) / 64), block(kFwdWaves * 64);
+  const int groups = (C + 63) / 64, seg = scan_seg_chunks(T, C, kFwdWaves * kFwdSteps, 3);
+  const int steps = seg * kFwdWaves * kFwdSteps, nseg = (T + steps - 1) / steps;
+  if (nseg > 1) {
+    hipLaunchKernelGGL(scan_fwd_map_kernel, dim3(groups, nseg - 1), dim3(kMapWaves * 64), 0, s, gates, eps, cck, steps,
+                       B, H);
+    hipLaunchKernelGGL(scan_fwd_carry_kernel, dim3(groups), dim3(64), 0, s, c0, eps, cck, steps, nseg, C);
+  }
+  const dim3 grid(groups, nseg), block(kFwdWaves * 64);
   if (sf == kBf16)
     hipLaunchKernelGGL((scan_fwd_kernel<kFwdWaves, kFwdSteps, kBf16>), grid, block, 0, s, gates, c0, eps, out, cck,
-                       T, B, H);
+                       T, B, H, seg);
   else if (sf == kF16)
     hipLaunchKernelGGL((scan_fwd_kernel<kFwdWaves, kFwdSteps, kF16>), grid, block, 0, s, gates, c0, eps, out, cck,
-                       T, B, H);
+                       T, B, H, seg);
   else
     hipLaunchKernelGGL((scan_fwd_kernel<kFwdWaves, kFwdSteps, kF32>), grid, block, 0, s, gates, c0, eps, out, cck,
-                       T, B, H);
+                       T, B, H, seg);
   HSL_HIP(hipGetLastError());
   timing_end(slot, s);
   return HSL_OK;
 }
 
+// Segments of the backward scan: db_part then holds [segments][B][4H].
+int scan_bwd_segments(int T, int B, int H, int* seg) {
+  *seg = scan_seg_chunks(T, (long)B * H, kBwdWaves * kBwdSteps, 5);
+  if (*seg < 1) return 1;
+  // a segment's steps are also the map kernel's 16 waves of whole 8-step groups
+  if (*seg * kBwdWaves * kBwdSteps < T) *seg = (*seg + 1) / 2 * 2;
+  const int steps = *seg * kBwdWaves * kBwdSteps;
+  return (T + steps - 1) / steps;
+}
+
 int scan_bwd(const float* gates, const float* c0, const float* cck, const void* dout, const float* dh_n,
-             const float* dc_n, float eps, float* dgates, double* db_part, float* dc0, int T, int B, int H,
-             hipStream_t s, int sf = kF32) {
+             const float* dc_n, float eps, float* dgates, double* db_part, float* dc0, int T, int B, int H, int seg,
+             int nseg, hipStream_t s, int sf = kF32) {
   const int C = B * H;
   if (C == 0) return HSL_OK;
   if (T == 0) {  // no steps: dc0 = dc_n through the clamp is not reached; all zero
@@ -406,16 +630,23 @@ int scan_bwd(const float* gates, const float* c0, const float* cck, const void* 
     return HSL_OK;
   }
   const int slot = timing_begin(kTimeScanBwd, s);
-  const dim3 grid((C + 63) / 64), block(kBwdWaves * 64);
+  const int groups = (C + 63) / 64, steps = nseg > 1 ? seg * kBwdWaves * kBwdSteps : 0;
+  if (nseg > 1) {
+    const auto map = sf == kBf16 ? scan_bwd_map_kernel<kBf16> : sf == kF16 ? scan_bwd_map_kernel<kF16> : scan_bwd_map_kernel<kF32>;
+    hipLaunchKernelGGL(map, dim3(groups, nseg - 1), dim3(kMapWaves * 64), 0, s, gates, cck, dout, dh_n, dc_n, eps,
+                       dgates, steps, T, B, H);
+    hipLaunchKernelGGL(scan_bwd_carry_kernel, dim3(groups), dim3(64), 0, s, dgates, steps, nseg, B, H);
+  }
+  const dim3 grid(groups, nseg), block(kBwdWaves * 64);
   if (sf == kBf16)
     hipLaunchKernelGGL((scan_bwd_kernel<kBwdWaves, kBwdSteps, kBf16>), grid, block, 0, s, gates, c0, cck, dout, dh_n,
-                       dc_n, eps, dgates, db_part, dc0, T, B, H);
+                       dc_n, eps, dgates, db_part, dc0, T, B, H, seg);
   else if (sf == kF16)
     hipLaunchKernelGGL((scan_bwd_kernel<kBwdWaves, kBwdSteps, kF16>), grid, block, 0, s, gates, c0, cck, dout, dh_n,
-                       dc_n, eps, dgates, db_part, dc0, T, B, H);
+                       dc_n, eps, dgates, db_part, dc0, T, B, H, seg);
   else
     hipLaunchKernelGGL((scan_bwd_kernel<kBwdWaves, kBwdSteps, kF32>), grid, block, 0, s, gates, c0, cck, dout, dh_n,
-                       dc_n, eps, dgates, db_part, dc0, T, B, H);
+                       dc_n, eps, dgates, db_part, dc0, T, B, H, seg);
   HSL_HIP(hipGetLastError());
   timing_end(slot, s);
   return HSL_OK;
@@ -423,7 +654,7 @@ int scan_bwd(const float* gates, const float* c0, const float* cck, const void* 
 
 struct ParWs {
   float* dgates;    // [T*B*4H]
-  double* db_part;  // [B*4H]
+  double* db_part;  // [segments][B*4H]
   float* gemm;
   size_t gemm_bytes;
 };
@@ -431,7 +662,8 @@ struct ParWs {
 size_t carve_par(void* ws, size_t cap, int T, int B, int D, int H, ParWs* o) {
   Carver c(ws, cap);
   o->dgates = c.take<float>((size_t)T * B * 4 * H);
-  o->db_part = c.take<double>((size_t)B * 4 * H);
+  int seg;
+  o->db_part = c.take<double>((size_t)scan_bwd_segments(T, B, H, &seg) * B * 4 * H);
   size_t g = gemm_ws_bytes_layout(4 * H, D, T * B, 1, 1, 0);
   const size_t g6 = gemm_ws_bytes_layout(T * B, D, 4 * H, 1, 0, 0);
   if (g6 > g) g = g6;
@@ -473,9 +705,11 @@ int par_bwd_impl(const void* dout, const float* dh_n, const float* dc_n, const v
     return HSL_OK;
   }
   if (!dout || !x || !gates || !c_ck) return fail(HSL_ERR_ARG, "%s: null pointer", fn);
-  HSL_CHECK(scan_bwd(gates, c0, c_ck, dout, dh_n, dc_n, eps, w.dgates, w.db_part, dc0, T, B, H, s,
+  int seg;
+  const int nseg = scan_bwd_segments(T, B, H, &seg);
+  HSL_CHECK(scan_bwd(gates, c0, c_ck, dout, dh_n, dc_n, eps, w.dgates, w.db_part, dc0, T, B, H, seg, nseg, s,
                      fmt < 0 ? kF32 : (fmt == 0 ? kBf16 : kF16)));
-  HSL_CHECK(bias_grads_from_parts(w.db_part, B, nullptr, nullptr, nullptr, db_ih, nullptr, nullptr, H, s));
+  HSL_CHECK(bias_grads_from_parts(w.db_part, B * nseg, nullptr, nullptr, nullptr, db_ih, nullptr, nullptr, H, s));
   const int TB = T * B;
   if (D > 0) {
     // dW_ih = dgates^T x, dx = dgates W_ih (B operands [K][N]; 16-bit ones pass as such)
@@ -517,8 +751,9 @@ int hsl_scan_bwd(const float* gates, const float* c0, const float* c_ck, const f
   HSL_CHECK(check_scan_dims(T, B, H));
   if (B > 0 && H > 0 && T > 0 && (!gates || !c_ck || !dout || !dgates))
     return fail(HSL_ERR_ARG, "hsl_scan_bwd: null pointer");
-  return scan_bwd(gates, c0, c_ck, dout, dh_n, dc_n, eps, dgates, db_part, dc0, T, B, H,
-                  static_cast<hipStream_t>(stream));
+  // one segment: db_part is [B][4H] here
+  return scan_bwd(gates, c0, c_ck, dout, dh_n, dc_n, eps, dgates, db_part, dc0, T, B, H, T / (kBwdWaves * kBwdSteps) + 1,
+                  1, static_cast<hipStream_t>(stream));
 }
 
 int hsl_par_fwd(const float* x, const float* c0, const float* w_ih, const float* b_ih, float eps, float* gates,

@@ -75,6 +75,17 @@ def test_small_shapes(dev, shape):
     check(*shape, dev, with_hx=True)
 
 
+@pytest.mark.parametrize("shape", [(385, 2, 12, 40),    # forward: 4 segments of one chunk, one step in the last
+                                   (321, 1, 8, 64),     # backward: 6 chunks, segments of two; forward: 3
+                                   (640, 3, 9, 70),     # whole chunks, a partial last channel group
+                                   (1027, 4, 16, 300),  # 19 channel groups: 9 and 9 segments, ragged T
+                                   (700, 5, 8, 1220),   # 96 channel groups, the most that are split: 2 segments
+                                   (700, 5, 8, 1230)])  # 97: not split
+def test_segmented_scans(dev, shape):
+    """Few channels: T runs as segments that start from states carried across them."""
+    check(*shape, dev, with_hx=True)
+
+
 def test_config1_parallel(dev):
     """configs[1] parallel: T128 B32 D256 H256."""
     check(128, 32, 256, 256, dev)
