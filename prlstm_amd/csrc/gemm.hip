@@ -3,9 +3,10 @@
 // Large C = A B^T products (at least 256 tiles of 256 x 256, no fp64 folding) and large
 // C = A^T B / A B products (weight gradients and dx, >= 8 GFLOP, split into fp32 runs of
 // <= 2048 k added in fp64)
-// run on the split-bf16 kernel of gemm_x6.hip (fp32 accuracy, 2.5x the matrix-core rate)
+// run on the split-bf16 kernel of gemm_x6.hip (fp32 accuracy, 2.5x the matrix-core rate),
+// smaller or ragged ones on its 128 x 128 tiles or on gemm_m6.hip,
 // unless hsl_set_split_products(0) selects the fp32 instruction for everything.
-// Products with M, N >= 64 run on the third core (gemm3_core.h): 128x256, 128x128 or
+// The other products with M, N >= 64 run on the third core (gemm3_core.h): 128x256, 128x128 or
 // 128x64 tiles, whichever is the largest that still gives two workgroups per CU, and
 // 128x64 tiles with fp64 folding for the long weight-gradient reductions.  Thinner
 // products (one side below 64, e.g. the [B,H] carries) use the first core's 32x32 tile.
@@ -215,6 +216,49 @@ int x6_longk_take(const GemmDesc& d, long max_planes) {
   if (s < 1 || (long)s * kSplitLongKRun < d.K) return 0;
   return s;
 }
+
+// Split count of a middle-sized split-bf16 product with at most `max_planes` planes (0: not
+// taken) and the kernel: *mid = whole 128 x 128 tiles of aligned rows (gemm_x6.hip), else
+// gemm_m6.hip.  A split is at most kSplitLongKRun deep when the sums are folded in fp32.
+bool vec_rows(const GemmDesc& d) {
+  return aligned16(d.A) && aligned16(d.B) && d.lda % 4 == 0 && d.ldb % 4 == 0;
+}
+int mid_take(const GemmDesc& d, long max_planes, int* mid) {
+  if (!split_products_mode()) return 0;
+  const long most = std::max(max_planes, 1L);
+  const bool fold = !(!d.trans_a && d.trans_b);
+  auto fits = [&](long s) { return s > 0 && (!fold || s * kSplitLongKRun >= d.K); };
+  *mid = 1;
+  long s = vec_rows(d) ? std::min<long>(gemm_x6_mid_splits(d.M, d.N, d.K, d.trans_a, d.trans_b), most) : 0;
+  if (fits(s)) return (int)s;
+  *mid = 0;
+  s = std::min<long>(gemm_m6_splits(d.M, d.N, d.K, d.trans_a, d.trans_b, d.lda, d.ldb), most);
+  return fits(s) ? (int)s : 0;
+}
+int mid_planes(int M, int N, int K, int trans_a, int trans_b) {
+  if (!split_products_mode()) return 0;
+  return std::max(gemm_x6_mid_splits(M, N, K, trans_a, trans_b),
+                  gemm_m6_splits(M, N, K, trans_a, trans_b, trans_a ? M : K, trans_b ? K : N));
+}
+int mid_run(const GemmDesc& d, int mid, float* partial, int splits, hipStream_t s, int* used) {
+  const auto run = [&](auto f, auto... more) {
+    return f(d.A, d.B, partial ? nullptr : d.bias, partial ? nullptr : d.C, partial, d.M, d.N, d.K, d.lda, d.ldb,
+             partial ? d.N : d.ldc, d.trans_a, d.trans_b, splits, s, used, more...);
+  };
+  return mid ? run(gemm_x6_run, 0, 1) : run(gemm_m6_run);
+}
+// The product on the middle-sized kernels with up to `planes` planes in ws; false: not taken.
+bool mid_product(const GemmDesc& d, long planes, void* ws, hipStream_t s, int* rc) {
+  int mid, used = 1;
+  const int sm = mid_take(d, planes, &mid);
+  if (!sm) return false;
+  float* const P = sm > 1 ? static_cast<float*>(ws) : nullptr;
+  *rc = mid_run(d, mid, P, sm, s, &used);
+  if (*rc == HSL_OK && P) *rc = splitk_reduce(P, used, d.bias, d.C, d.M, d.N, d.ldc, s);
+  return true;
+}
+// A product that the large tiles would run on their masked instances.
+bool ragged(const GemmDesc& d) { return !gemm_x6_full(d.M, d.N, d.K, d.trans_a, d.trans_b, vec_rows(d)); }
 }  // namespace
 
 size_t gemm_ws_bytes_layout(int M, int N, int K, int acc64, int trans_a, int trans_b) {
@@ -223,20 +267,25 @@ size_t gemm_ws_bytes_layout(int M, int N, int K, int acc64, int trans_a, int tra
     const int s = gemm_x6_longk_splits(M, N, K);
     if (s > 1) need = std::max(need, sizeof(float) * (size_t)s * M * N);
   }
+  const int m = mid_planes(M, N, K, trans_a, trans_b);
+  if (m > 1) need = std::max(need, sizeof(float) * (size_t)m * M * N);
   return need;
 }
 
 int gemm_tn_planes(int M, int N, int K) {
   int s = gemm_pick_splits(M, N, K, 1);
   if (split_products_mode()) s = std::max(s, gemm_x6_longk_splits(M, N, K));
-  return s;
+  return std::max(s, mid_planes(M, N, K, 1, 0));
 }
 
 int gemm_partials(const GemmDesc& d, float* partials, int splits, hipStream_t s, int* used) {
   HSL_CHECK(check_desc(d));
+  int mid;
+  if (const int sm = ragged(d) ? mid_take(d, splits, &mid) : 0) return mid_run(d, mid, partials, sm, s, used);
   if (const int sx = x6_longk_take(d, splits))
     return gemm_x6_run(d.A, d.B, nullptr, nullptr, partials, d.M, d.N, d.K, d.lda, d.ldb, d.N, d.trans_a, 0, sx, s,
                        used);
+  if (const int sm = mid_take(d, splits, &mid)) return mid_run(d, mid, partials, sm, s, used);
   return dispatch(pick_tile(d.M, d.N, d.acc64), d, partials, std::min(splits, gemm_pick_splits(d.M, d.N, d.K, d.acc64)), s,
                   used);
 }
@@ -244,10 +293,15 @@ int gemm_partials(const GemmDesc& d, float* partials, int splits, hipStream_t s,
 int gemm_run(const GemmDesc& d, void* ws, size_t ws_bytes, hipStream_t s) {
   HSL_CHECK(check_desc(d));
   if (d.M == 0 || d.N == 0) return HSL_OK;
-  if (!d.trans_a && d.trans_b && !d.acc64 && split_products_mode() && gemm_x6_applies(d.M, d.N, d.K))
-    return gemm_x6_run(d.A, d.B, d.bias, d.C, nullptr, d.M, d.N, d.K, d.lda, d.ldb, d.ldc, 0, 1, 1, s, nullptr);
   // planes the workspace holds (one split needs none: it writes C directly)
   const long planes = ws ? (long)(ws_bytes / (sizeof(float) * (size_t)d.M * d.N)) : 0;
+  const bool mid_first = ragged(d);
+  if (mid_first) {
+    int rc;
+    if (mid_product(d, planes, ws, s, &rc)) return rc;
+  }
+  if (!d.trans_a && d.trans_b && !d.acc64 && split_products_mode() && gemm_x6_applies(d.M, d.N, d.K))
+    return gemm_x6_run(d.A, d.B, d.bias, d.C, nullptr, d.M, d.N, d.K, d.lda, d.ldb, d.ldc, 0, 1, 1, s, nullptr);
   if (const int sx = x6_longk_take(d, planes > 1 ? planes : 1)) {
     if (sx == 1)
       return gemm_x6_run(d.A, d.B, d.bias, d.C, nullptr, d.M, d.N, d.K, d.lda, d.ldb, d.ldc, d.trans_a, 0, 1, s,
@@ -257,6 +311,8 @@ int gemm_run(const GemmDesc& d, void* ws, size_t ws_bytes, hipStream_t s) {
     HSL_CHECK(gemm_x6_run(d.A, d.B, nullptr, nullptr, P, d.M, d.N, d.K, d.lda, d.ldb, d.N, d.trans_a, 0, sx, s, &used));
     return splitk_reduce(P, used, d.bias, d.C, d.M, d.N, d.ldc, s);
   }
+  int rc;
+  if (!mid_first && mid_product(d, planes, ws, s, &rc)) return rc;
   const Tile t = pick_tile(d.M, d.N, d.acc64);
   int splits = gemm_pick_splits(d.M, d.N, d.K, d.acc64);
   if (splits > 1) splits = actual_splits(t, d.K, splits);
@@ -292,7 +348,7 @@ int gemm_run_b16(const GemmDesc& d, int fmt, float* widen, void* ws, size_t ws_b
   HSL_CHECK(check_desc(d));
   if (d.trans_b) return fail(HSL_ERR_ARG, "gemm_run_b16: B must be [K][N]");
   if (d.M == 0 || d.N == 0) return HSL_OK;
-  if (fmt == 0) {  // a bf16 value is one bf16 piece: the split kernel reads it as it is
+  if (fmt == 0 && !ragged(d)) {  // a bf16 value is one bf16 piece: the split kernel reads it as it is
     const long planes = ws ? (long)(ws_bytes / (sizeof(float) * (size_t)d.M * d.N)) : 0;
     if (const int sx = x6_longk_take(d, planes > 1 ? planes : 1)) {
       if (sx == 1)

@@ -22,7 +22,8 @@
 // rule is therefore simple: a non-finite element of A makes its row of C NaN, one of B
 // its column (v - v0 is NaN or infinite, and so are the later pieces); a finite value
 // beyond the bf16 range (|v| > 3.3895e38) rounds to v0 = +-inf and counts as non-finite.
-// hsl_set_split_products(0) gives the IEEE results of the fp32 instruction instead.
+// hsl_set_split_products(0) gives the IEEE results of the fp32 instruction instead.  The
+// 128 x 128 tiles compute a part whose result holds a NaN again with that instruction.
 //
 // Workgroup = 8 waves.  The projection uses 256 x 256 tiles (2 x 4 waves of 128 x 64, i.e.
 // 4 x 2 fragments of 32 x 32); the long-K products use 256 x 128 tiles (4 x 2 waves of
@@ -40,6 +41,7 @@
 // written transposed, each row's k-pair as one 32-bit word per piece.  A bf16 B operand
 // (a half-precision module's x or W_ih) is its own single piece: only it is staged and
 // three products per k-step are issued (X6OperandB16).
+#include <algorithm>
 #include <type_traits>
 
 #include "gemm_core.h"
@@ -62,6 +64,7 @@ struct X6Shape {
   static constexpr int TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
   static constexpr int PA = BM * kLDK, PB = BN * kLDK;  // one piece of A / of B
   static constexpr int BUF = 3 * (PA + PB);             // pieces 0-2 of A, then of B
+  static constexpr bool kIeee = BM == 128;              // non-finite operands give the fp32 instruction's results
   static constexpr size_t LDS = 2 * BUF * sizeof(unsigned short);
   static_assert(WM * WN * 64 == kThreads && TM % 32 == 0 && TN % 32 == 0, "wave layout");
   static_assert(LDS <= 160 * 1024, "LDS");
@@ -70,6 +73,11 @@ struct X6Shape {
 using ShapeProj = X6Shape<256, 256, 2, 4, 0>;
 // A^T B: 256 x 128 tiles, 8 waves of 64 x 64, folded every 4 slices (64 k)
 using ShapeWgrad = X6Shape<256, 128, 4, 2, 4>;
+// Products with too few of those tiles, on whole 128 x 128 tiles: 8 waves of 32 x 64, one
+// register set and at most 128 registers, so that two workgroups share a CU and cover each
+// other's fragment reads and barriers (4 waves of 64 x 64, with a third less LDS traffic,
+// had nothing to cover them: 4096 x 1024 x 256 20-24 us against 17.9, fp32 instruction 26).
+using ShapeMid = X6Shape<128, 128, 4, 2, 4>;
 
 struct X6Args {
   const float* A;
@@ -292,7 +300,7 @@ __device__ __forceinline__ void x6_tile(const X6Args& g, int m0, int n0, unsigne
   // shorter than a load's latency under load (one set: configs[4] dW_ih at 38% MFMA busy,
   // waves waiting 54% of their cycles; two sets took configs[4] from 2.54 to 2.42 ms per
   // step, three to 2.42-2.43).  The projection shape has no registers to spare.
-  constexpr int NSET = S::FOLD ? 3 : 1;
+  constexpr int NSET = S::FOLD && S::BM == 256 ? 3 : 1;
   using OpA = X6Operand<FULL, AKC, S::BM, NSET>;
   using OpB = std::conditional_t<BP == 1, X6OperandB16<FULL, NSET>, X6Operand<FULL, BKC, S::BN, NSET>>;
   constexpr int NPP = BP == 1 ? 3 : 6;  // piece products per k-step
@@ -431,6 +439,41 @@ __device__ __forceinline__ void x6_tile(const X6Args& g, int m0, int n0, unsigne
     if (it + 1 < nk) iteration(it + 1, std::integral_constant<int, 2>{});
   }
 
+  if constexpr (S::kIeee) {
+    // a NaN in the wave's results: its part again on the fp32 instruction (IEEE results for
+    // non-finite operands, as these products had before they ran on split pieces)
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < S::FM; ++i)
+#pragma unroll
+      for (int j = 0; j < S::FN; ++j) {
+        const f16v& res = S::FOLD ? tot[S::FOLD ? i : 0][S::FOLD ? j : 0] : acc[i][j];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) nan = nan || res[r] != res[r];
+      }
+    if (__any(nan)) {
+#pragma unroll
+      for (int i = 0; i < S::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < S::FN; ++j) {
+          f16v& res = S::FOLD ? tot[S::FOLD ? i : 0][S::FOLD ? j : 0] : acc[i][j];
+          const int m = min(m0 + wm * S::TM + 32 * i + r32, g.M - 1), n = min(n0 + wn * S::TN + 32 * j + r32, g.N - 1);
+          f16v sum = f16v{}, run = f16v{};
+          for (int k = kbeg; k < kend; k += 2) {
+            const int kk = k + half;
+            const float a = kk < kend ? g.A[AKC ? (size_t)m * g.lda + kk : (size_t)kk * g.lda + m] : 0.f;
+            const float b = kk < kend ? g.B[BKC ? (size_t)n * g.ldb + kk : (size_t)kk * g.ldb + n] : 0.f;
+            run = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, run, 0, 0, 0);
+            if (S::FOLD && (k + 2 - kbeg) % 64 == 0) {
+              sum += run;
+              run = f16v{};
+            }
+          }
+          res = sum + run;
+        }
+    }
+  }
+
   float* outp = g.partial ? g.out + (size_t)blockIdx.z * g.M * g.N : g.out;
   const int ldo = g.partial ? g.N : g.ldc;
   if constexpr (FULL) {
@@ -510,7 +553,7 @@ __device__ __forceinline__ void x6_tile(const X6Args& g, int m0, int n0, unsigne
 // (M, N multiples of the tile, K and the split length of 16, aligned operands); chosen
 // per launch, so the unmasked kernel carries no edge code.  AKC / BKC: operand k-contiguous.
 template <class S, bool FULL, bool AKC, bool BKC, int BP>
-__global__ __launch_bounds__(kThreads) void gemm_x6_kernel(X6Args g) {
+__global__ __launch_bounds__(kThreads, S::BM == 128 ? 4 : 1) void gemm_x6_kernel(X6Args g) {
   extern __shared__ unsigned short x6_smem[];
   int tm, tn;
   if constexpr (S::FOLD) {
@@ -550,10 +593,50 @@ long x6_tiles(int M, int N) {
 }
 }  // namespace
 
+namespace {
+// Whole 128 x 128 tiles and enough work that they beat the smaller ones of gemm_m6.hip
+// (measured: 1024 x 256 x 4096 A^T B 29 against 33 us, 4096 x 256 x 1024 A B 25 against 28,
+// 2304 x 3072 x 512 A B^T 51 against 64).
+bool x6_mid(int M, int N, int K) {
+  return M % ShapeMid::BM == 0 && N % ShapeMid::BN == 0 && K % kBK == 0 && (double)M * N * K >= 2.5e8;
+}
+// k-splits of a long-K product: a split's time is the rounds its workgroups run in times its
+// depth, and each split writes and reads a plane.  Filling the chip is not enough: 48 tiles of
+// 256 x 128 in 6 splits are 288 workgroups, two rounds on 256 CUs (3072 x 512 x 12288: 297 us,
+// in 10 splits 226 us; 3072 x 768 x 2304: 101 -> 75 us).  us_k: us per k of a workgroup on its
+// own CU; us_k2: of two that share one (0 where they do not fit).
+int x6_pick_splits(long tiles, int M, int N, int K, double us_k, double us_k2, long least) {
+  const long most = std::max(least, std::min<long>(64, K / 128));
+  long best = least;
+  double best_us = 0.0;
+  for (long s = least; s <= most; ++s) {
+    const long wgs = tiles * s, slots = us_k2 > 0.0 ? 512 : 256, rest = wgs % slots;
+    const double full = us_k2 > 0.0 ? us_k2 : us_k, last = rest == 0 ? 0.0 : rest <= 256 ? us_k : full;
+    const double us = (wgs / slots * full + last) * ((K + s - 1) / s) + (s > 1 ? 3.0 + s * (double)M * N * 8.0 / 4e6 : 0.0);
+    if (s == least || us < best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return (int)best;
+}
+}  // namespace
+
+int gemm_x6_mid_splits(int M, int N, int K, int trans_a, int trans_b) {
+  if ((trans_a && trans_b) || !x6_mid(M, N, K)) return 0;
+  if (!trans_a && trans_b) return 1;
+  return x6_pick_splits(x6_tiles<ShapeMid>(M, N), M, N, K, 0.05, 0.077, (K + kSplitLongKRun - 1) / kSplitLongKRun);
+}
+
 bool gemm_x6_applies(int M, int N, int K) {
   // one tile per CU at least (256 x 256, or else 256 x 128), and enough k to amortise the
   // tile's setup
   return (x6_tiles<ShapeProj>(M, N) >= 256 || x6_tiles<ShapeWgrad>(M, N) >= 256) && K >= 32;
+}
+
+bool gemm_x6_full(int M, int N, int K, int trans_a, int trans_b, bool vec) {
+  const bool proj = !trans_a && trans_b && x6_tiles<ShapeProj>(M, N) >= 256;
+  return vec && M % 256 == 0 && N % (proj ? ShapeProj::BN : ShapeWgrad::BN) == 0 && K % kBK == 0;
 }
 
 int gemm_x6_longk_splits(int M, int N, int K) {
@@ -564,12 +647,8 @@ int gemm_x6_longk_splits(int M, int N, int K) {
   using S = ShapeWgrad;
   if (M < S::BM || N < S::BN || K < 2 * kBK || 2.0 * M * N * K < 8e9) return 0;
   const long tiles = (long)((M + S::BM - 1) / S::BM) * ((N + S::BN - 1) / S::BN);
-  long s = (256 + tiles - 1) / tiles;
-  const long by_run = (K + kSplitLongKRun - 1) / kSplitLongKRun;
-  if (by_run > s) s = by_run;
-  if (s > K / kBK) s = K / kBK;
-  if (s > 64) s = 64;
-  return s < 1 ? 1 : (int)s;
+  const long by_run = std::min<long>(64, (K + kSplitLongKRun - 1) / kSplitLongKRun);
+  return x6_pick_splits(tiles, M, N, K, 0.096, 0.0, by_run);
 }
 
 int gemm_x6_wgrad_fin(const float* A, const float* B, float* C, const float* a_group, int group_rows,
@@ -606,7 +685,8 @@ int gemm_x6_wgrad_fin(const float* A, const float* B, float* C, const float* a_g
 }
 
 int gemm_x6_run(const float* A, const void* B, const float* bias, float* C, float* partial, int M, int N, int K,
-                int lda, int ldb, int ldc, int trans_a, int trans_b, int splits, hipStream_t s, int* used, int b_bf16) {
+                int lda, int ldb, int ldc, int trans_a, int trans_b, int splits, hipStream_t s, int* used, int b_bf16,
+                int mid) {
   if (M <= 0 || N <= 0 || K <= 0) return fail(HSL_ERR_ARG, "gemm_x6: empty product");
   if (trans_a && trans_b) return fail(HSL_ERR_ARG, "gemm_x6: layout not supported");
   if (b_bf16 && trans_b) return fail(HSL_ERR_ARG, "gemm_x6: a bf16 B must be [K][N] (trans_b = 0)");
@@ -630,7 +710,13 @@ int gemm_x6_run(const float* A, const void* B, const float* bias, float* C, floa
   if (used) *used = n;
   const bool vec = aligned16(A) && aligned16(B) && lda % 4 == 0 && ldb % 4 == 0;
   g.out_vec = aligned16(g.out) && (partial ? N % 4 == 0 : ldc % 4 == 0) && (g.bias == nullptr || aligned16(g.bias));
-  if (b_bf16 && trans_a)
+  if (mid && !trans_a && trans_b)
+    x6_launch<ShapeMid, true, true>(g, vec, n, s);
+  else if (mid && trans_a)
+    x6_launch<ShapeMid, false, false>(g, vec, n, s);
+  else if (mid)
+    x6_launch<ShapeMid, true, false>(g, vec, n, s);
+  else if (b_bf16 && trans_a)
     x6_launch<ShapeWgrad, false, false, 1>(g, vec, n, s);  // dgates^T x with a bf16 x
   else if (b_bf16)
     x6_launch<ShapeWgrad, true, false, 1>(g, vec, n, s);  // dgates W_ih with a bf16 W_ih

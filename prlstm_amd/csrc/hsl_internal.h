@@ -112,13 +112,26 @@ int gemm_pick_splits(int M, int N, int K, int acc64);
 // the parity tolerance against fp64 (the CPU's own fp32 product: 1.12x); 2048 gives 1.08x.
 constexpr int kSplitLongKRun = 2048;
 bool gemm_x6_applies(int M, int N, int K);  // C = A B^T products (input projection)
+// Whether a product the large tiles apply to is whole tiles of aligned rows.  Their masked
+// instances read element by element (4099 x 4100 x 257 A B^T: 189 us, gemm_m6.hip 86 us), so
+// they only serve operands beyond the other kernel's 32-bit offsets.
+bool gemm_x6_full(int M, int N, int K, int trans_a, int trans_b, bool vec);
 int gemm_x6_longk_splits(int M, int N, int K);  // C = A^T B or A B: split count, 0 = not taken
 // Split-bf16 product (gemm_x6.hip): any layout but trans_a = trans_b = 1;
 // with partial != nullptr the k-splits go to planes [used][M][N] (no bias).
 // b_bf16: B holds bf16 values (one piece each; trans_b = 0 only), three products per step.
 int gemm_x6_run(const float* A, const void* B, const float* bias, float* C, float* partial, int M, int N, int K,
                 int lda, int ldb, int ldc, int trans_a, int trans_b, int splits, hipStream_t s, int* used,
-                int b_bf16 = 0);
+                int b_bf16 = 0, int mid = 0);
+// The same kernel on 128 x 128 tiles (mid = 1), for products of whole tiles that are too small
+// for the others: the k-splits to run, 0 = not taken.  Needs 16-byte aligned rows.
+int gemm_x6_mid_splits(int M, int N, int K, int trans_a, int trans_b);
+// Middle-sized split-bf16 products (gemm_m6.hip; every layout but trans_a = trans_b = 1, any
+// alignment): the k-splits to run, 0 = not taken; with partial != nullptr the splits go to
+// planes [used][M][N] (no bias).
+int gemm_m6_splits(int M, int N, int K, int trans_a, int trans_b, int lda, int ldb);
+int gemm_m6_run(const float* A, const float* B, const float* bias, float* C, float* partial, int M, int N, int K,
+                int lda, int ldb, int ldc, int trans_a, int trans_b, int splits, hipStream_t s, int* used);
 // dW = A^T B written with its finalisation (one split of the split-bf16 kernel): row r of
 // C = a_group[r / group_rows] * (A^T B)[r], and per group the fp64 sum of W . (A^T B) in
 // parts[group][*parts] of dotp.  *parts = 0: the shape does not qualify and nothing ran.

@@ -230,3 +230,53 @@ def test_split_products_exact_on_representable_sums(dev, split_products, layout,
     cx6, c32 = _both(a.float().to(dev), b.float().to(dev), None, M, N, K, ta=ta, tb=int(layout.startswith("abt")))
     assert torch.equal(cx6, exact)
     assert torch.equal(c32, exact)
+
+
+MIDDLE = [(64, 96, 1024), (65, 1024, 95), (129, 1000, 65), (200, 64, 1931), (1000, 63, 203), (333, 65, 700),
+          (131, 33, 1430), (700, 650, 2603), (1027, 130, 64),              # gemm_m6.hip: edges of tiles and slices
+          (128, 128, 16384), (256, 384, 2560), (1024, 256, 1040)]          # whole 128 x 128 tiles
+LAYOUTS = [(0, 0), (0, 1), (1, 0)]
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("M,N,K", MIDDLE)
+@pytest.mark.parametrize("pad", [0, 1])
+def test_middle_split_products(dev, split_products, M, N, K, ta, tb, pad):
+    """Middle-sized and ragged products on split pieces, with and without 16-byte aligned rows:
+    the fp32 bound against fp64, an rms error not above the fp32 kernel's (5% for the sampling
+    noise of the rms), and nothing written past the rows of C."""
+    print(f"middle split products M={M} N={N} K={K} ta={ta} tb={tb} pad={pad}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randn(*((K, M + pad) if ta else (M, K + pad)), generator=g)
+    b = torch.randn(*((N, K + pad) if tb else (K, N + pad)), generator=g) * 0.1
+    bias = torch.randn(N, generator=g)
+    c6, c32 = _both(a.to(dev), b.to(dev), bias.to(dev), M, N, K, ta=ta, tb=tb)
+    assert not torch.equal(c6, c32)  # two different kernels ran
+    av = (a[:, :M].t() if ta else a[:, :K]).double()
+    bv = (b[:, :K].t() if tb else b[:, :N]).double()
+    ref = av @ bv + bias.double()
+    scale = av.abs() @ bv.abs() + bias.double().abs()
+    e6, e32 = (c6 - ref).abs() / scale, (c32 - ref).abs() / scale
+    assert float(e6.max()) <= 2e-6 * K ** 0.5
+    assert float(e6.pow(2).mean().sqrt()) <= 1.05 * float(e32.pow(2).mean().sqrt())
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("M,N,K", [(200, 100, 700), (256, 256, 4096)])
+def test_middle_split_products_non_finite(dev, split_products, M, N, K, ta, tb):
+    """Non-finite and out-of-bf16-range operands give the fp32 instruction's results: the same
+    NaN, +inf and -inf elements, and finite elements within the fp32 bound of each other."""
+    print(f"non-finite M={M} N={N} K={K} ta={ta} tb={tb}", flush=True)
+    g = torch.Generator().manual_seed(K)
+    a = torch.randn(M, K, generator=g)
+    b = torch.randn(N, K, generator=g)
+    a[3, 5], a[40, 7], a[77, K - 1], a[199, 0] = float("inf"), float("-inf"), float("nan"), 3.4e38
+    b[9, 2], b[99, K - 1] = float("inf"), float("nan")
+    A = (a.t().contiguous() if ta else a).to(dev)
+    B = (b if tb else b.t().contiguous()).to(dev)
+    c6, c32 = _both(A, B, None, M, N, K, ta=ta, tb=tb)
+    for what in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(what(c6), what(c32)), what
+    ok = torch.isfinite(c32)
+    scale = (a.double().abs() @ b.double().abs().t())[ok]
+    assert bool(((c6 - c32)[ok].abs() <= 4e-6 * K ** 0.5 * scale).all())

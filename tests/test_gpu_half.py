@@ -150,7 +150,7 @@ def test_gemm_b16_unaligned_rows(dev):
 
 
 @pytest.mark.parametrize("fmt", [0, 1])
-@pytest.mark.parametrize("T,B,D,H", [(32, 4, 16, 24), (4096, 16, 256, 1024)])
+@pytest.mark.parametrize("T,B,D,H", [(32, 4, 16, 24), (700, 2, 16, 40), (250, 9, 300, 700), (4096, 16, 256, 1024)])
 def test_parallel_backward_16bit_operands_equal_widened(dev, fmt, T, B, D, H):
     """hsl_par_bwd_b16 reads the 16-bit x and W_ih itself: a bf16 value is one bf16 piece,
     so the split-product kernel issues three products per k-step instead of six (at
