@@ -86,7 +86,8 @@ int hsl_set_exchange_scope(int mode);
  * backend calls torch.nn.functional.linear). */
 int hsl_set_split_products(int on);
 /* Which path the last hsl_rec_fwd / hsl_rec_bwd in this process (on any host
- * thread; autograd runs the backward on its own thread) used: 1 = per-step,
+ * thread; autograd runs the backward on its own thread) used: 1 = per-step (one
+ * step of at most 8 rows in a launch of its own included),
  * 2 = persistent, 3 = the persistent kernels that hold W_hh in the registers of
  * 256 workgroups (512 < H <= 2048). */
 int hsl_last_recurrent_path(void);

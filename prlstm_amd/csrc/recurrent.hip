@@ -23,6 +23,7 @@
 // A_b[i][0], B from lane 4b+j is B_b[0][j], result lane 4b+j, reg i holds D_b[i][j].
 // With cbsz=4, abid=0 every block uses block 0's A (lanes 0-3).
 #include <algorithm>
+#include <map>
 #include <mutex>
 #include <cstdlib>
 #include <type_traits>
@@ -2057,6 +2058,120 @@ __global__ __launch_bounds__(XT >= 0 ? 512 : 256, 1) void rec_bwd_persistent(PBw
   }
 }
 
+// ---------------------------------------------------------------------------------
+// one time step of a few rows (a stream that carries its state from call to call)
+// ---------------------------------------------------------------------------------
+// The whole step in one launch (_torch.py:96, :111-120 at T = 1): wave = one unit, whose four
+// gate rows of W_ih and W_hh are read once and multiplied with the BT batch rows; the lanes'
+// partial sums meet in a butterfly, and lane b runs row b's cell.  Bound by reading the two
+// weight matrices (6.3 MB at D = 256, H = 512) with all the chip's CUs, where a persistent
+// launch loads W_hh into the registers of one XCD and needs its hand-off slots filled first:
+// B = 1: 14.5 us (fill 2, kernel 12.5), here 5 us.
+struct OneStepArgs {
+  const float *x, *h0, *c0, *w_ih, *w_hh, *b_ih, *b_hh, *a;
+  float *h_save, *c_save, *gact, *tanh_c;
+  int* err;  // the call's error words, cleared
+  int B, D, H;
+  int vec;   // rows of x, h0 and both weights are 16-byte aligned
+};
+constexpr int kOneStepRows = 8;  // batch rows up to which the step runs this way
+
+// acc[g][b] += scale_g * (row of gate g) . (row b), over K columns
+template <int BT, bool VEC>
+__device__ __forceinline__ void one_step_dot(float (&acc)[4][BT], const float* __restrict__ w, const float* __restrict__ v,
+                                             const float (&scale)[4], int u, int H, int K, int B) {
+  constexpr int E = VEC ? 4 : 1;
+  const int lane = threadIdx.x & 63;
+  float sum[4][BT];
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int b = 0; b < BT; ++b) sum[g][b] = 0.f;
+  for (int k = E * lane; k < K; k += 64 * E) {
+    float wv[4][E];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float* const p = w + (size_t)(g * H + u) * K + k;
+      if constexpr (VEC) {
+        const f4 q = *reinterpret_cast<const f4*>(p);
+#pragma unroll
+        for (int e = 0; e < E; ++e) wv[g][e] = q[e];
+      } else {
+        wv[g][0] = *p;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < BT; ++b) {
+      const float* const p = v + (size_t)(b < B ? b : 0) * K + k;
+      float xv[E];
+      if constexpr (VEC) {
+        const f4 q = *reinterpret_cast<const f4*>(p);
+#pragma unroll
+        for (int e = 0; e < E; ++e) xv[e] = q[e];
+      } else {
+        xv[0] = *p;
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int e = 0; e < E; ++e) sum[g][b] = __builtin_fmaf(wv[g][e], xv[e], sum[g][b]);
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int b = 0; b < BT; ++b) acc[g][b] = __builtin_fmaf(scale[g], sum[g][b], acc[g][b]);
+}
+
+template <int BT>
+__global__ __launch_bounds__(256) void rec_fwd_one_step(OneStepArgs p) {
+  const int lane = threadIdx.x & 63;
+  const int u = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (blockIdx.x == 0 && threadIdx.x < 64) p.err[threadIdx.x] = 0;
+  if (u >= p.H) return;
+  const int B = p.B, D = p.D, H = p.H;
+  float ag[4];
+  const float one[4] = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+  for (int g = 0; g < 4; ++g) ag[g] = p.a[g];
+  float acc[4][BT];
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int b = 0; b < BT; ++b) acc[g][b] = 0.f;
+  if (p.vec) {
+    one_step_dot<BT, true>(acc, p.w_ih, p.x, one, u, H, D, B);
+    if (p.h0) one_step_dot<BT, true>(acc, p.w_hh, p.h0, ag, u, H, H, B);
+  } else {
+    one_step_dot<BT, false>(acc, p.w_ih, p.x, one, u, H, D, B);
+    if (p.h0) one_step_dot<BT, false>(acc, p.w_hh, p.h0, ag, u, H, H, B);
+  }
+  float z[4] = {0.f, 0.f, 0.f, 0.f};  // lane b: row b's pre-activations
+#pragma unroll
+  for (int b = 0; b < BT; ++b)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float s = acc[g][b];
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+      z[g] = lane == b ? s : z[g];
+    }
+  if (lane >= BT || lane >= B) return;
+  const size_t e = (size_t)lane * H + u, plane = (size_t)B * H;
+  const float h_in = p.h0 ? p.h0[e] : 0.f, c_in = p.c0 ? p.c0[e] : 0.f;
+  float act[4];
+#pragma unroll
+  for (int g = 0; g < 4; ++g) act[g] = sigmoid_f((z[g] + p.b_ih[g * H + u]) + ag[g] * p.b_hh[g * H + u]);
+  const float c = act[1] * c_in + act[0] * act[2];
+  const float tc = tanh_f(c);
+  p.h_save[e] = h_in;
+  p.c_save[e] = c_in;
+  p.h_save[plane + e] = act[3] * tc;
+  p.c_save[plane + e] = c;
+  p.tanh_c[e] = tc;
+  *reinterpret_cast<f4*>(p.gact + 4 * e) = f4{act[0], act[1], act[2], act[3]};
+}
+
 #include "rec_wide.h"
 #include "rec_wide_fwd.h"
 #include "rec_wide_bwd32.h"
@@ -2082,12 +2197,29 @@ int pick_kq(int H) {
   return 0;
 }
 
-template <class K>
-int max_resident(K kernel, int threads, int* out) {
+// Resident workgroups per CU of a kernel with its launch's LDS, asked of the runtime once per
+// kernel and device (the answer is a property of the code object; a call plans twice, for its
+// workspace and for its launch).
+int resident(const void* kernel, int threads, size_t lds, int* out) {
+  DeviceInfo di;
+  HSL_CHECK(device_info(&di));
+  static std::mutex mu;
+  static std::map<std::pair<int, const void*>, int> known;
+  std::lock_guard<std::mutex> lock(mu);
+  const auto it = known.find({di.device, kernel});
+  if (it != known.end()) {
+    *out = it->second;
+    return HSL_OK;
+  }
   int occ = 0;
-  HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, threads, kFwdLdsBytes));
+  HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, threads, lds));
+  known[{di.device, kernel}] = occ;
   *out = occ;
   return HSL_OK;
+}
+template <class K>
+int max_resident(K kernel, int threads, int* out) {
+  return resident(reinterpret_cast<const void*>(kernel), threads, kFwdLdsBytes, out);
 }
 
 // Weight-gradient waves in the persistent backward: on unless HSL_FUSED_WGRAD=0.
@@ -2128,16 +2260,13 @@ int bwd_resident_ws(int xt, int* occ) {
   int o = 0;
   switch (xt) {
     case -1:
-      HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, rec_bwd_persistent<KQ, -1, 2>, 256,
-                                                           bwd_lds_bytes(-1, true)));
+      HSL_CHECK(resident((const void*)rec_bwd_persistent<KQ, -1, 2>, 256, bwd_lds_bytes(-1, true), &o));
       break;
     case 0:
-      HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, rec_bwd_persistent<KQ, 0, WS>, 512,
-                                                           bwd_lds_bytes(0, WS)));
+      HSL_CHECK(resident((const void*)rec_bwd_persistent<KQ, 0, WS>, 512, bwd_lds_bytes(0, WS), &o));
       break;
     default:
-      HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&o, rec_bwd_persistent<KQ, 2, WS>, 512,
-                                                           bwd_lds_bytes(2, WS)));
+      HSL_CHECK(resident((const void*)rec_bwd_persistent<KQ, 2, WS>, 512, bwd_lds_bytes(2, WS), &o));
       break;
   }
   *occ = o;
@@ -2257,9 +2386,8 @@ const void* wide_kernel(bool bwd) {
 }
 template <int U>
 int wide_occupancy(bool bwd, bool pad, int* occ) {
-  HSL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, pad ? wide_kernel<U, true>(bwd) : wide_kernel<U, false>(bwd),
-                                                       256, bwd ? wide_bwd_lds<U>() : wide_fwd_lds<U>()));
-  return HSL_OK;
+  return resident(pad ? wide_kernel<U, true>(bwd) : wide_kernel<U, false>(bwd), 256,
+                  bwd ? wide_bwd_lds<U>() : wide_fwd_lds<U>(), occ);
 }
 
 // The width of the wide kernels that hold a hidden size (units per k block / 4), 0 = none.
@@ -2413,6 +2541,11 @@ size_t carve_fwd(void* ws, size_t cap, int T, int B, int H, FwdNeeds nd, FwdWs* 
     o->part = c.take<float>(sp > 1 ? (size_t)sp * B * 4 * H : 0);
   }
   return c.off;
+}
+
+// One step of at most kOneStepRows rows runs in a launch of its own (unless a path is forced).
+bool one_step(int T, int B, int D) {
+  return T == 1 && B >= 1 && B <= kOneStepRows && D > 0 && recurrent_path_mode() == 0;
 }
 
 // The workspace parts of a forward call with this plan; the fused projection needs a
@@ -2629,7 +2762,9 @@ size_t hsl_rec_fwd_ws_bytes(int T, int B, int D, int H) {
   FwdNeeds nd;  // every part when the path cannot be planned (no device)
   PersistentPlan pl;
   WidePlan wp;
-  if (B > 0 && H > 0 && plan_persistent(B, H, D, false, &pl) == HSL_OK && plan_wide(B, H, false, &wp) == HSL_OK)
+  if (one_step(T, B, D))
+    nd.xch = nd.gih = nd.step = nd.wide = false;
+  else if (B > 0 && H > 0 && plan_persistent(B, H, D, false, &pl) == HSL_OK && plan_wide(B, H, false, &wp) == HSL_OK)
     nd = fwd_needs(pl, wp, true);
   return carve_fwd(nullptr, 0, T, B, H, nd, &w);
 }
@@ -2642,6 +2777,22 @@ int hsl_rec_fwd(const float* x, const float* h0, const float* c0, const float* w
   if (B == 0 || H == 0) return HSL_OK;
   if (!w_hh || !b_hh || !a || !h_save || !c_save || (T > 0 && (!x || !w_ih || !b_ih || !gact || !tanh_c)))
     return fail(HSL_ERR_ARG, "hsl_rec_fwd: null pointer");
+  if (one_step(T, B, D)) {
+    FwdWs w;
+    FwdNeeds nd;
+    nd.xch = nd.gih = nd.step = nd.wide = false;
+    const size_t need = carve_fwd(ws, ws_bytes, T, B, H, nd, &w);
+    if (!ws || ws_bytes < need) return fail(HSL_ERR_ARG, "hsl_rec_fwd: workspace %zu bytes, need %zu", ws_bytes, need);
+    const bool vec = D % 4 == 0 && H % 4 == 0 && aligned16(x) && aligned16(w_ih) && aligned16(w_hh) && (!h0 || aligned16(h0));
+    const OneStepArgs oa{x, h0, c0, w_ih, w_hh, b_ih, b_hh, a, h_save, c_save, gact, tanh_c, w.err, B, D, H, vec ? 1 : 0};
+    const auto kernel = B == 1 ? rec_fwd_one_step<1> : B == 2 ? rec_fwd_one_step<2> : B <= 4 ? rec_fwd_one_step<4> : rec_fwd_one_step<8>;
+    const int slot = timing_begin(kTimeStepFwd, s);
+    hipLaunchKernelGGL(kernel, dim3((H + 3) / 4), dim3(256), 0, s, oa);
+    HSL_HIP(hipGetLastError());
+    timing_end(slot, s);
+    note_recurrent_path(1);
+    return HSL_OK;
+  }
   PersistentPlan pl;
   HSL_CHECK(plan_persistent(B, H, D, false, &pl));
   WidePlan wp;

@@ -166,6 +166,16 @@ def test_batch_over_several_launches(dev, T, B, D, H):
     assert prlstm_amd.last_recurrent_path() == 2
 
 
+@pytest.mark.parametrize("B,D,H", [(1, 256, 512), (1, 1, 1), (2, 7, 33), (3, 260, 1026), (5, 64, 128), (8, 30, 300)])
+@pytest.mark.parametrize("with_hx", [True, False])
+def test_one_step_of_few_rows(dev, B, D, H, with_hx):
+    """T = 1 with at most 8 rows: one launch, unit by unit (16-byte or 4-byte loads), and
+    what it saves feeds the backward.  A ninth row takes the other paths."""
+    check(1, B, D, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=with_hx, fwd_path=1)
+    if H == 300:
+        check(1, B + 1, D, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=with_hx, fwd_path=2)
+
+
 def test_batch_beyond_the_launches(dev):
     check(2, 129, 16, 512, dev, 0, a=[0.3, 0.5, 0.1, 0.2], fwd_path=1)
 
