@@ -90,12 +90,14 @@ def load():
 
 
 def ptr(t):
-    """Device pointer of a tensor (or NULL for None)."""
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    """Device pointer of a tensor (or NULL for None), as the int that a void* argument takes
+    (0 is NULL too: an empty tensor)."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_of(device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current HIP stream of the device, as the int that a void* argument takes."""
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 def call(name, *args):
