@@ -479,7 +479,7 @@ __device__ __forceinline__ void word_put(float* base, unsigned off, float v) {
     __hip_atomic_store(u, __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A lane's N (1, 2, 4 or 8) words inside a block of 64 lanes: with N == 1 word 0 of
+// A lane's N (1 or even) words inside a block of 64 lanes: with N == 1 word 0 of
 // lane l is at l; otherwise word j is at 128*(j/2) + 2*l + j%2, so a lane's words pair
 // up into 8-byte loads and stores and the 64 lanes of a pair are contiguous.
 template <int N>
@@ -756,7 +756,7 @@ __device__ __forceinline__ void rec_fwd_body(const PFwdArgs& p, int grp, int wg,
       // block and each lane reads its row back: an eighth of the cache-line requests.
       // At configs[2] the slice is in registers 9.3-9.7 us after launch instead of 11.2
       // (the rest is the 32 MiB that the eight XCDs' copies of W_hh read).
-      constexpr int KC = KQ < 64 ? KQ : 64;  // k per staging pass
+      constexpr int KC = KQ < 64 ? KQ : KQ % 64 ? 32 : 64;  // k per staging pass
       constexpr int LPR = KC / 4, RPI = 64 / LPR, PITCH = KC + 4;
       float* const stg = fwd_wstage(xin) + q * 64 * PITCH;
       static_assert(4 * 64 * PITCH * sizeof(float) <= kFwdWStageBytes, "staging fits");
@@ -2196,6 +2196,12 @@ int pick_kq(int H) {
   if (H <= 512) return 128;
   return 0;
 }
+// The forward's quarters can also be 96 wide (256 < H <= 384): a step issues KQ products in a
+// row on each SIMD, 0.43 us of its time at KQ = 128, and columns past H are multiplied like
+// the others.  Forward, us, 128 wide / 96 wide: T100 B10 D80 H300 149 / 134, T200 B32 D256 H384
+// 302 / 269, T100 B32 D300 H257 207 / 179.  The backward keeps 128: its products come in
+// 64-column groups, two on the busiest wave at either width.
+int pick_kq_fwd(int H) { return H > 256 && H <= 384 ? 96 : pick_kq(H); }
 
 // Resident workgroups per CU of a kernel with its launch's LDS, asked of the runtime once per
 // kernel and device (the answer is a property of the code object; a call plans twice, for its
@@ -2249,11 +2255,14 @@ int fwd_resident(int xp, int* occ) {
   }
 }
 
-// One launch at KQ = 128 adds the weight-gradient products straight to the long sums (WS = 1):
+// One launch at H > 384 adds the weight-gradient products straight to the long sums (WS = 1):
 // there the additions of the window sums lengthen the launch by 0.6% (519 -> 522 us at
 // T256 B32 D256 H512).  Several launches, whose dW_hh would otherwise be less accurate than
-// the per-step path's, and smaller KQ, where they cost nothing measurable, take WS = 2.
-int wgrad_form(int kq, int launches) { return !split_products_mode() ? 0 : kq == 128 && launches == 1 ? 1 : 2; }
+// the per-step path's, and smaller H, where they cost little (training step at T200 B32 D256
+// H384 678 -> 684 us, dW_hh's relative error 4.7e-7 -> 1.8e-7), take WS = 2.
+int wgrad_form(int kq, int H, int launches) {
+  return !split_products_mode() ? 0 : kq == 128 && H > 384 && launches == 1 ? 1 : 2;
+}
 
 template <int KQ, int WS>
 int bwd_resident_ws(int xt, int* occ) {
@@ -2292,7 +2301,7 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
   *pl = PersistentPlan{};
   const int mode = recurrent_path_mode();
   if (mode == 1) return HSL_OK;
-  const int kq = pick_kq(H);
+  const int kq = bwd ? pick_kq(H) : pick_kq_fwd(H);
   if (kq == 0 || B < 1) return HSL_OK;
   DeviceInfo di;
   HSL_CHECK(device_info(&di));
@@ -2308,7 +2317,7 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
   // x rows with 16-byte loads
   if (!bwd && fused_xproj_enabled()) p.XP = D > 0 && D <= 256 && D % 4 == 0;
   p.XS = kXprojSplit && split_products_mode();
-  p.WS = wgrad_form(kq, 1);
+  p.WS = wgrad_form(kq, H, 1);
   int occ = 0;
   for (;;) {
     if (bwd) {
@@ -2324,6 +2333,7 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
         case 16: HSL_CHECK(fwd_resident<16>(xp, &occ)); break;
         case 32: HSL_CHECK(fwd_resident<32>(xp, &occ)); break;
         case 64: HSL_CHECK(fwd_resident<64>(xp, &occ)); break;
+        case 96: HSL_CHECK(fwd_resident<96>(xp, &occ)); break;
         default: HSL_CHECK(fwd_resident<128>(xp, &occ)); break;
       }
     }
@@ -2339,7 +2349,7 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
       p.NGX = (p.gpl + di.num_xcds - 1) / di.num_xcds * di.num_xcds;
       p.grid = p.NGX * p.NW;
       p.ok = p.launches <= (mode == 2 ? 1 : kMaxGroupLaunches);
-      p.WS = wgrad_form(kq, p.launches);
+      p.WS = wgrad_form(kq, H, p.launches);
     }
     if (p.ok || fit > 0 || (p.XT < 0 && !p.XP)) break;
     p.XT = -1;  // retry without the weight-gradient / projection waves
@@ -2518,7 +2528,7 @@ size_t carve_fwd(void* ws, size_t cap, int T, int B, int H, FwdNeeds nd, FwdWs* 
   Carver c(ws, cap);
   *o = FwdWs{};
   o->err = c.take<int>(64);
-  const int kq = pick_kq(H);
+  const int kq = pick_kq_fwd(H);
   if (nd.xch && kq) {
     const size_t ng = (size_t)(B + 3) / 4;
     o->hwords = ng * (size_t)(4 * kq / kUnits);
@@ -2838,6 +2848,7 @@ int hsl_rec_fwd(const float* x, const float* h0, const float* c0, const float* w
         case 16: launch_fwd_persistent<16>(pa, pl.grid, xp, s); break;
         case 32: launch_fwd_persistent<32>(pa, pl.grid, xp, s); break;
         case 64: launch_fwd_persistent<64>(pa, pl.grid, xp, s); break;
+        case 96: launch_fwd_persistent<96>(pa, pl.grid, xp, s); break;
         default: launch_fwd_persistent<128>(pa, pl.grid, xp, s); break;
       }
       HSL_HIP(hipGetLastError());

@@ -154,6 +154,15 @@ def test_device_scope_exchange(dev, shape):
     check(*shape, dev, 2, a=[0.6, 0.2, 0.9, 0.4])
 
 
+@pytest.mark.parametrize("H", [256, 257, 300, 352, 383, 384, 385])
+@pytest.mark.parametrize("B,D,scope", [(5, 12, 0), (33, 270, 1)])
+def test_forward_quarters_of_96(dev, H, B, D, scope):
+    """The forward's k quarters are 96 wide for 256 < H <= 384, on both sides of each line, with
+    and without the fused projection and in either hand-off scope."""
+    prlstm_amd.set_exchange_scope(scope)
+    check(7, B, D, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=True, fwd_path=2)
+
+
 @pytest.mark.parametrize("T,B,D,H", [(9, 33, 20, 512),    # 9 groups: launches of 5 and 4
                                      (3, 128, 16, 512),   # the most launches: 4 of 8 groups
                                      (9, 66, 270, 300),   # D > 256: separate dW_ih, dgates of both launches
