@@ -191,7 +191,7 @@ int check_desc(const GemmDesc& d) {
 
 int gemm_pick_splits(int M, int N, int K, int acc64) {
   const long tiles = tile_count(pick_tile(M, N, acc64), M, N);
-  if (tiles >= kFill || K < 1024) return 1;
+  if (tiles < 1 || tiles >= kFill || K < 1024) return 1;  // (no tiles: an empty product)
   int s = (int)((2 * kFill + tiles - 1) / tiles);  // aim for ~1024 workgroups
   const int max_by_k = K / 512;                    // keep >= 512 k per split
   if (s > max_by_k) s = max_by_k;

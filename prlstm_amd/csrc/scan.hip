@@ -573,7 +573,7 @@ __global__ __launch_bounds__(64) void scan_bwd_carry_kernel(float* dgates, int s
 //   T = 256, 16 groups (H = 256): 12.5, 22.1 / 14.6, 23.1 -> at least `least` chunks
 int scan_seg_chunks(int T, long C, int chunk, int least) {
   const int groups = (int)((C + 63) / 64), nchunks = (T + chunk - 1) / chunk;
-  if (groups > 96 || nchunks < least) return nchunks;
+  if (groups < 1 || groups > 96 || nchunks < least) return nchunks;  // no channels (B or H of 0): nothing to split
   const int nseg = std::min(nchunks, 256 / groups);
   return nseg < 2 ? nchunks : (nchunks + nseg - 1) / nseg;
 }

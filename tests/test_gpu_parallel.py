@@ -86,6 +86,21 @@ def test_segmented_scans(dev, shape):
     check(*shape, dev, with_hx=True)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T", [3, 300])
+def test_empty_batch(dev, T, dtype):
+    """A batch of no sequences: empty outputs and zero parameter gradients, for short sequences
+    and for those long enough to be cut into segments."""
+    m = prlstm_amd.HeadStartLSTM(8, 16, parallel=True).to(dev, dtype)
+    x = torch.zeros(T, 0, 8, device=dev, dtype=dtype, requires_grad=True)
+    out, (h_n, c_n) = m(x)
+    assert out.shape == (T, 0, 16) and h_n.shape == c_n.shape == (1, 0, 16)
+    out.sum().backward()
+    assert x.grad.shape == x.shape
+    for p in (m.weight_ih_l0, m.bias_ih_l0):
+        assert torch.count_nonzero(p.grad) == 0 and torch.isfinite(p.grad).all()
+
+
 def test_config1_parallel(dev):
     """configs[1] parallel: T128 B32 D256 H256."""
     check(128, 32, 256, 256, dev)

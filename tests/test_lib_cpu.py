@@ -63,6 +63,11 @@ def test_workspace_queries():
     assert lib.hsl_par_bwd_f64_ws_bytes(4096, 16, 256, 1024) >= 4096 * 16 * 4 * 1024 * 8
     for f in (lib.hsl_rec_fwd_f64_ws_bytes, lib.hsl_rec_bwd_f64_ws_bytes, lib.hsl_par_bwd_f64_ws_bytes):
         assert f(-1, 1, 1, 1) == 0
+    # an empty batch or no hidden units: a size like any other, also where T is long enough to
+    # be cut into segments (whose count is planned from the channels)
+    for f in (lib.hsl_par_bwd_ws_bytes, lib.hsl_par_bwd_b16_ws_bytes):
+        for T in (1, 256, 257, 300, 16384):
+            assert f(T, 0, 8, 16) < 4096 and f(T, 2, 8, 0) < 4096 + 4 * T * 2 * 8, T
     # parallel mode keeps c every 8th step: ceil(T/8) carry-in rows, then c_n
     for T, rows in ((1, 2), (7, 2), (8, 2), (9, 3), (128, 17), (4096, 513), (0, 1), (-1, 0)):
         assert lib.hsl_scan_ck_rows(T) == rows, (T, lib.hsl_scan_ck_rows(T))
