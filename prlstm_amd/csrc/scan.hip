@@ -390,6 +390,14 @@ __global__ __launch_bounds__(NW * 64) void scan_bwd_kernel(
 // forward's 20 bytes per element and 20 of the backward's 36 once more.
 constexpr int kMapWaves = 16;
 
+// A product of gates in a map.  A segment's underflows (0.5 after 150 steps) and is then held
+// at the smallest denormal, unless a factor is 0 (eps = 0): an infinite state stays infinite
+// across a segment, as it does through the scan kernels' 8-step maps, where 0 * inf would make
+// it NaN.  A finite state x moves by at most 1.4e-45 |x|.
+__device__ __forceinline__ float map_prod(float a, float b) {
+  return fmaxf(a * b, fminf(fminf(a, b), __uint_as_float(1u)));
+}
+
 // Forward map of segment blockIdx.y (never the last one, so every step is below T): wave w
 // composes the w-th part of its `steps` steps in groups of 8.
 __global__ __launch_bounds__(kMapWaves * 64) void scan_fwd_map_kernel(const float* __restrict__ gates, float eps,
@@ -417,7 +425,7 @@ __global__ __launch_bounds__(kMapWaves * 64) void scan_fwd_map_kernel(const floa
     for (int s = 0; s < kCkSteps; ++s) {
       const float f = fmaxf(sigmoid_f(z[1][s]), eps);
       const float bb = fmaxf(sigmoid_prod_f(z[0][s], z[2][s]), eps);
-      A = f * A;
+      A = map_prod(f, A);
       V = f * V + bb;
     }
   }
@@ -429,7 +437,7 @@ __global__ __launch_bounds__(kMapWaves * 64) void scan_fwd_map_kernel(const floa
 #pragma unroll
     for (int u = 0; u < kMapWaves; ++u) {
       const float2 m = sAV[u][lane];
-      A = m.x * A;
+      A = map_prod(m.x, A);
       V = m.x * V + m.y;
     }
     float* const row = cck + ((size_t)blockIdx.y * steps / kCkSteps + 1) * C + ch;
@@ -517,7 +525,7 @@ __global__ __launch_bounds__(kMapWaves * 64) void scan_bwd_map_kernel(
       if (t < T) {
         const float f = t + 1 < T ? (s + 1 < kCkSteps ? fg[s + 1 < kCkSteps ? s + 1 : 0] : fn) : 0.f;
         V = ev[s] + f * V;
-        A = f * A;
+        A = map_prod(f, A);
       }
     }
   }
@@ -529,7 +537,7 @@ __global__ __launch_bounds__(kMapWaves * 64) void scan_bwd_map_kernel(
 #pragma unroll
     for (int u = kMapWaves - 1; u >= 0; --u) {
       const float2 m = sAV[u][lane];
-      A = m.x * A;
+      A = map_prod(m.x, A);
       V = m.x * V + m.y;
     }
     float* const row = dgates + (size_t)ts * gstride + (size_t)b * 4 * H + j;

@@ -86,6 +86,39 @@ def test_segmented_scans(dev, shape):
     check(*shape, dev, with_hx=True)
 
 
+@pytest.mark.parametrize("T,B,D,H,bf", [(1500, 1, 8, 64, -3.0),   # 12 and 12 segments of 128 steps, f near 0.05
+                                        (700, 6, 4, 1024, 0.0)])  # 96 channel groups: 384 steps, f near 0.5
+def test_segmented_scans_carry_infinite_states(dev, T, B, D, H, bf):
+    """A segment's map multiplies hundreds of forget gates, whose product underflows; an infinite
+    c0 stays infinite all the same (out = o, c_n = inf) and an infinite gradient reaches dc0 with
+    its sign, as through the step-by-step recurrence.  Other channels are untouched by it."""
+    torch.manual_seed(T)
+    m = prlstm_amd.HeadStartLSTM(D, H, parallel=True).to(dev)
+    with torch.no_grad():
+        m.bias_ih_l0[H:2 * H] = bf
+    x = torch.randn(T, B, D, device=dev)
+    h0, c0 = torch.zeros(1, B, H, device=dev), torch.rand(1, B, H, device=dev)
+    with torch.no_grad():
+        want, (_, want_c) = m(x, (h0, c0))
+        c_inf = c0.clone()
+        c_inf[0, 0, 5] = float("inf")
+        out, (_, c_n) = m(x, (h0, c_inf))
+        o = torch.sigmoid(x[:, 0].double() @ m.weight_ih_l0[3 * H + 5].double() + m.bias_ih_l0[3 * H + 5].double())
+    assert c_n[0, 0, 5] == float("inf")
+    assert (out[:, 0, 5].double() - o).abs().max() < 1e-6
+    out[:, 0, 5], c_n[0, 0, 5] = want[:, 0, 5], want_c[0, 0, 5]
+    assert torch.equal(out, want) and torch.equal(c_n, want_c)
+    c0.requires_grad_(True)
+    out, (_, c_n) = m(x, (h0, c0))
+    w = torch.ones_like(c_n)
+    w[0, 0, 7], w[0, -1, 9] = float("inf"), float("-inf")
+    c_n.backward(w)
+    assert c0.grad[0, 0, 7] == float("inf") and c0.grad[0, -1, 9] == float("-inf")
+    rest = c0.grad.clone()
+    rest[0, 0, 7] = rest[0, -1, 9] = 0.0
+    assert torch.isfinite(rest).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T", [3, 300])
 def test_empty_batch(dev, T, dtype):
