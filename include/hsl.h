@@ -157,9 +157,12 @@ int hsl_rec_fwd(const float* x, const float* h0, const float* c0,
  * the parts that must start empty with a fill kernel.  Shapes whose workspace
  * exceeds 4 MiB are rejected with HSL_ERR_UNSUPPORTED; the persistent path with
  * the input projection fused (H <= 512, D <= 256, D % 4 == 0, 16-byte aligned x,
- * a batch that fits the chip) needs well under 1 MiB.  Every call on one device
+ * a batch of one launch) needs well under 1 MiB.  A larger batch (H <= 512) is
+ * accepted where the per-step path's buffers fit, among them 4H*H weights (so
+ * never at H = 512), and runs the persistent launches where theirs fit too, else
+ * the per-step path.  Every call on one device
  * shares that device's scratch: calls that overlap on one device (two streams,
- * two threads) race.  Results equal hsl_rec_fwd's bit for bit. */
+ * two threads) race.  Results equal, bit for bit, hsl_rec_fwd's on the path that ran. */
 int hsl_rec_fwd_noalloc(const float* x, const float* h0, const float* c0,
                         const float* w_ih, const float* w_hh, const float* b_ih,
                         const float* b_hh, const float* a,

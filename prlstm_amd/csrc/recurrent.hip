@@ -2744,44 +2744,11 @@ int scratch_address(void** out) {
   *out = g_scratch_addr[dev];
   return HSL_OK;
 }
-}  // namespace
-}  // namespace hsl
 
-using namespace hsl;
-
-extern "C" {
-
-int hsl_device_errors(int* flags, int clear, void* stream) {
-  if (!flags) return fail(HSL_ERR_ARG, "hsl_device_errors: null pointer");
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  unsigned v = 0;
-  HSL_HIP(hipMemcpyFromSymbolAsync(&v, HIP_SYMBOL(g_device_errors), sizeof(v), 0, hipMemcpyDeviceToHost, s));
-  HSL_HIP(hipStreamSynchronize(s));
-  if (clear && v) {
-    hipLaunchKernelGGL(clear_device_errors_kernel, dim3(1), dim3(1), 0, s);
-    HSL_HIP(hipGetLastError());
-    HSL_HIP(hipStreamSynchronize(s));
-  }
-  *flags = static_cast<int>(v);
-  return HSL_OK;
-}
-
-size_t hsl_rec_fwd_ws_bytes(int T, int B, int D, int H) {
-  if (T < 0 || B < 0 || D < 0 || H < 0) return 0;
-  FwdWs w;
-  FwdNeeds nd;  // every part when the path cannot be planned (no device)
-  PersistentPlan pl;
-  WidePlan wp;
-  if (one_step(T, B, D))
-    nd.xch = nd.gih = nd.step = nd.wide = false;
-  else if (B > 0 && H > 0 && plan_persistent(B, H, D, false, &pl) == HSL_OK && plan_wide(B, H, false, &wp) == HSL_OK)
-    nd = fwd_needs(pl, wp, true);
-  return carve_fwd(nullptr, 0, T, B, H, nd, &w);
-}
-
-int hsl_rec_fwd(const float* x, const float* h0, const float* c0, const float* w_ih, const float* w_hh,
-                const float* b_ih, const float* b_hh, const float* a, float* h_save, float* c_save, float* gact,
-                float* tanh_c, void* ws, size_t ws_bytes, int T, int B, int D, int H, void* stream) {
+// hsl_rec_fwd; per_step: the per-step path whatever the shape.
+int rec_fwd(const float* x, const float* h0, const float* c0, const float* w_ih, const float* w_hh, const float* b_ih,
+            const float* b_hh, const float* a, float* h_save, float* c_save, float* gact, float* tanh_c, void* ws,
+            size_t ws_bytes, int T, int B, int D, int H, bool per_step, void* stream) {
   HSL_CHECK(check_dims(T, B, D, H));
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (B == 0 || H == 0) return HSL_OK;
@@ -2804,9 +2771,9 @@ int hsl_rec_fwd(const float* x, const float* h0, const float* c0, const float* w
     return HSL_OK;
   }
   PersistentPlan pl;
-  HSL_CHECK(plan_persistent(B, H, D, false, &pl));
   WidePlan wp;
-  if (!pl.ok) HSL_CHECK(plan_wide(B, H, false, &wp));
+  if (!per_step) HSL_CHECK(plan_persistent(B, H, D, false, &pl));
+  if (!per_step && !pl.ok) HSL_CHECK(plan_wide(B, H, false, &wp));
   if (recurrent_path_mode() == 2 && !pl.ok && !wp.ok)
     return fail(HSL_ERR_UNSUPPORTED, "persistent path does not fit (B=%d H=%d)", B, H);
   const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
@@ -2914,6 +2881,47 @@ int hsl_rec_fwd(const float* x, const float* h0, const float* c0, const float* w
   note_recurrent_path(1);
   return HSL_OK;
 }
+}  // namespace
+}  // namespace hsl
+
+using namespace hsl;
+
+extern "C" {
+
+int hsl_device_errors(int* flags, int clear, void* stream) {
+  if (!flags) return fail(HSL_ERR_ARG, "hsl_device_errors: null pointer");
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  unsigned v = 0;
+  HSL_HIP(hipMemcpyFromSymbolAsync(&v, HIP_SYMBOL(g_device_errors), sizeof(v), 0, hipMemcpyDeviceToHost, s));
+  HSL_HIP(hipStreamSynchronize(s));
+  if (clear && v) {
+    hipLaunchKernelGGL(clear_device_errors_kernel, dim3(1), dim3(1), 0, s);
+    HSL_HIP(hipGetLastError());
+    HSL_HIP(hipStreamSynchronize(s));
+  }
+  *flags = static_cast<int>(v);
+  return HSL_OK;
+}
+
+size_t hsl_rec_fwd_ws_bytes(int T, int B, int D, int H) {
+  if (T < 0 || B < 0 || D < 0 || H < 0) return 0;
+  FwdWs w;
+  FwdNeeds nd;  // every part when the path cannot be planned (no device)
+  PersistentPlan pl;
+  WidePlan wp;
+  if (one_step(T, B, D))
+    nd.xch = nd.gih = nd.step = nd.wide = false;
+  else if (B > 0 && H > 0 && plan_persistent(B, H, D, false, &pl) == HSL_OK && plan_wide(B, H, false, &wp) == HSL_OK)
+    nd = fwd_needs(pl, wp, true);
+  return carve_fwd(nullptr, 0, T, B, H, nd, &w);
+}
+
+int hsl_rec_fwd(const float* x, const float* h0, const float* c0, const float* w_ih, const float* w_hh,
+                const float* b_ih, const float* b_hh, const float* a, float* h_save, float* c_save, float* gact,
+                float* tanh_c, void* ws, size_t ws_bytes, int T, int B, int D, int H, void* stream) {
+  return rec_fwd(x, h0, c0, w_ih, w_hh, b_ih, b_hh, a, h_save, c_save, gact, tanh_c, ws, ws_bytes, T, B, D, H, false,
+                 stream);
+}
 
 int hsl_rec_fwd_noalloc(const float* x, const float* h0, const float* c0, const float* w_ih, const float* w_hh,
                         const float* b_ih, const float* b_hh, const float* a, float* h_save, float* c_save,
@@ -2928,23 +2936,28 @@ int hsl_rec_fwd_noalloc(const float* x, const float* h0, const float* c0, const 
   if (pl.XP && !x_aligned) pl.XP = false;
   FwdWs w;
   size_t need = carve_fwd(nullptr, 0, T, B, H, fwd_needs(pl, wp, x_aligned), &w);
-  if (pl.launches > 1) {  // a batch beyond one launch is held to the per-step path's buffers
+  // a batch beyond one persistent launch is accepted where the per-step path's buffers fit, and
+  // runs that path where the buffers of its launches do not
+  bool per_step = false;
+  if (pl.launches > 1) {
     FwdNeeds step;
     step.xch = step.wide = false;
-    need = std::max(need, carve_fwd(nullptr, 0, T, B, H, step, &w));
+    per_step = need > kNoAllocScratchBytes;
+    need = carve_fwd(nullptr, 0, T, B, H, step, &w);
   }
   if (need > kNoAllocScratchBytes)
     return fail(HSL_ERR_UNSUPPORTED,
                 "hsl_rec_fwd_noalloc: T=%d B=%d D=%d H=%d needs %zu bytes of scratch, more than the %zu bytes of "
-                "its static scratch buffer (the persistent path with the input projection fused -- H <= 512, "
-                "D <= 256, D %% 4 == 0, 16-byte aligned x -- needs well under 1 MiB); call hsl_rec_fwd with a "
-                "workspace instead",
-                T, B, D, H, need, kNoAllocScratchBytes);
+                "its static scratch buffer%s (the persistent path in one launch with the input projection fused -- "
+                "H <= 512, D <= 256, D %% 4 == 0, 16-byte aligned x -- needs well under 1 MiB); call hsl_rec_fwd with "
+                "a workspace instead",
+                T, B, D, H, need, kNoAllocScratchBytes,
+                pl.launches > 1 ? ", counting the per-step path's buffers for a batch beyond one launch" : "");
   void* ws = nullptr;
   HSL_CHECK(scratch_address(&ws));
   TimingSuppress no_events;
-  return hsl_rec_fwd(x, h0, c0, w_ih, w_hh, b_ih, b_hh, a, h_save, c_save, gact, tanh_c, ws, kNoAllocScratchBytes, T,
-                     B, D, H, stream);
+  return rec_fwd(x, h0, c0, w_ih, w_hh, b_ih, b_hh, a, h_save, c_save, gact, tanh_c, ws, kNoAllocScratchBytes, T, B, D,
+                 H, per_step, stream);
 }
 
 size_t hsl_rec_bwd_ws_bytes_for(int T, int B, int D, int H, int with_dx) {

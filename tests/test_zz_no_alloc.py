@@ -134,3 +134,36 @@ def test_rec_fwd_noalloc_rejects_shapes_beyond_its_scratch(dev):
     torch.cuda.synchronize()
     for n in o:  # nothing ran: the outputs still hold their NaN fill
         assert torch.isnan(o[n]).all(), n
+
+
+@pytest.mark.parametrize("T,path", [(1, 2), (6, 2), (7, 1)])
+def test_rec_fwd_noalloc_accepts_batches_of_several_launches(dev, T, path):
+    """B = 256 at H = 128 runs as two persistent launches, whose hand-off slots (1 MiB) lie beside
+    the gate buffer when D > 256.  Where both fit the scratch they run; one step further only the
+    per-step path's buffers fit (3.94 MB of 4.19), which the call accepts as ever and runs; either
+    way the outputs are those of hsl_rec_fwd on that path, bit for bit."""
+    B, D, H = 256, 300, 128
+    print(f"noalloc T={T} B={B} D={D} H={H}", flush=True)
+    i = _inputs(T, B, D, H, dev, seed=T)
+    got = _outputs(T, B, H, dev)
+    _lib.call("hsl_rec_fwd_noalloc", *_args(i, got), T, B, D, H, _lib.stream_of(dev))
+    torch.cuda.synchronize()
+    assert _lib.last_recurrent_path() == path
+    prev = _lib.load().hsl_set_recurrent_path(1 if path == 1 else 0)
+    try:
+        ref = _reference(i, T, B, D, H, dev)
+    finally:
+        _lib.load().hsl_set_recurrent_path(prev)
+    _assert_equal(got, ref, f"T={T}")
+    _lib.check_errors(dev)
+
+
+@pytest.mark.parametrize("T,B,D,H", [(8, 256, 300, 128),   # the gate buffer alone fills the scratch
+                                     (2, 64, 16, 512)])    # the per-step path's W_hh does
+def test_rec_fwd_noalloc_rejects_batches_of_several_launches(dev, T, B, D, H):
+    i, o = _inputs(T, B, D, H, dev, seed=3), _outputs(T, B, H, dev)
+    lib = _lib.load()
+    assert lib.hsl_rec_fwd_noalloc(*_args(i, o), T, B, D, H, _lib.stream_of(dev)) == 2
+    assert b"static scratch" in lib.hsl_last_error()
+    torch.cuda.synchronize()
+    assert torch.isnan(o["h_save"]).all()
