@@ -2445,8 +2445,14 @@ int plan_wide(int B, int H, bool bwd, WidePlan* pl) {
 // six 32-term products, or 512 single products.  Longer sequences share the 8 chunks, so
 // a chunk spans ceil(T / 8) steps (at T = 2048 with the fp32 products: 1024 single
 // products per running sum, which the long-sequence test checks against the parity bar).
-int wgrad_chunks(int T, bool ws) {
-  const int span = ws ? 256 : 128;
+// A batch of several launches takes 128 steps with the window products too, which keeps
+// dW_hh as accurate as the per-step path's product (folded every 64 k over at most 2048 k)
+// that the launches stand in for: relative error against 64 bits, mean of 16 inputs, per-step /
+// spans of 256 / of 128: T250 B100 D64 H512 1.80e-7 / 1.87e-7 / 1.72e-7, T256 B128 D256 H512
+// 2.04e-7 / 2.12e-7 / 1.99e-7, T200 B96 D128 H256 1.72e-7 / 1.85e-7 / 1.73e-7 (the second plane
+// of each group costs 0.7 to 2% of the step: 3825 -> 3902 us at T256 B128 D256 H512).
+int wgrad_chunks(int T, bool ws, int launches) {
+  const int span = ws && launches == 1 ? 256 : 128;
   const int c = (T + span - 1) / span;
   return c < 1 ? 1 : (c > 8 ? 8 : c);
 }
@@ -2601,7 +2607,7 @@ size_t gemm_region_bytes(int T, int B, int D, int H) {
   if (pick_kq(H) && fused_wgrad_enabled()) {  // planes of the fused weight gradients
     const size_t ng = (B + 3) / 4;
     // sized for the fp32 products' shorter chunks, whatever the mode is now
-    const size_t wg = sizeof(float) * wgrad_chunks(T, false) * ng * 4 * H * H +
+    const size_t wg = sizeof(float) * wgrad_chunks(T, false, 1) * ng * 4 * H * H +
                       (D <= 256 ? sizeof(float) * ng * 4 * H * D : 0);
     if (wg > need) need = wg;
   }
@@ -3015,7 +3021,7 @@ int hsl_rec_bwd(const float* dout, const float* dh_n, const float* dc_n, const f
   float* const wph = w.gemm;
   float* wpx = nullptr;
   if (fused) {
-    const int nch = wgrad_chunks(T, pl.WS);
+    const int nch = wgrad_chunks(T, pl.WS, pl.launches);
     wts = ((T + nch - 1) / nch + 7) / 8 * 8;  // whole 8-step windows per plane
     nsplit = (T + wts - 1) / wts * pl.NG;
     wpx = wph + (size_t)nsplit * 4 * H * H;

@@ -185,6 +185,34 @@ def test_one_step_of_few_rows(dev, B, D, H, with_hx):
         check(1, B + 1, D, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=with_hx, fwd_path=2)
 
 
+def test_weight_gradient_of_several_launches_is_as_accurate_as_per_step(dev):
+    """Sequences of more than 128 steps in several launches: the fused dW_hh is no further from
+    the fp64 module's than that of the per-step path, which the launches stand in for."""
+    T, B, D, H = 250, 100, 64, 512
+    print(f"dW_hh of several launches T={T} B={B} D={D} H={H}", flush=True)
+    torch.manual_seed(1)
+    ref = prlstm_amd.HeadStartLSTM(D, H).to(dev).double()
+    with torch.no_grad():
+        ref.a.copy_(0.5 * torch.rand(4))
+    m = prlstm_amd.HeadStartLSTM(D, H).to(dev)
+    with torch.no_grad():
+        for p, q in zip(ref.parameters(), m.parameters()):
+            q.copy_(p)
+            p.copy_(q)
+    x, dout = torch.randn(T, B, D, device=dev), torch.randn(T, B, H, device=dev)
+    ref(x.double())[0].backward(dout.double())
+    want = ref.weight_hh_l0.grad
+    err = {}
+    for mode, path in ((0, 2), (1, 1)):
+        prlstm_amd.set_recurrent_path(mode)
+        m.zero_grad()
+        m(x)[0].backward(dout)
+        assert prlstm_amd.last_recurrent_path() == path
+        err[path] = float((m.weight_hh_l0.grad.double() - want).norm() / want.norm())
+    print(err)
+    assert err[2] <= err[1] <= 1e-6
+
+
 def test_batch_beyond_the_launches(dev):
     check(2, 129, 16, 512, dev, 0, a=[0.3, 0.5, 0.1, 0.2], fwd_path=1)
 
