@@ -219,15 +219,32 @@ int x6_longk_take(const GemmDesc& d, long max_planes) {
 
 // Split count of a middle-sized split-bf16 product with at most `max_planes` planes (0: not
 // taken) and the kernel: *mid = whole 128 x 128 tiles of aligned rows (gemm_x6.hip), else
-// gemm_m6.hip.  A split is at most kSplitLongKRun deep when the sums are folded in fp32.
+// gemm_m6.hip.  The weight gradients and dx run in splits of at most kSplitLongKRun; C = A B^T
+// needs none (relative error at K = 16384 3.3e-7 in one split, the fp32 kernel's 2.3e-6).
 bool vec_rows(const GemmDesc& d) {
   return aligned16(d.A) && aligned16(d.B) && d.lda % 4 == 0 && d.ldb % 4 == 0;
+}
+// Products that stay on the fp32 kernel (gemm3_core.h): whole tiles of it, few enough that a
+// CU has one workgroup or none, where its shorter slices (no split, no fold) are the lower
+// latency.  us, fp32 kernel / split pieces:
+//   one split, up to 256 tiles of 128 x 64: A B^T 256 x 512 x 64 5.8 / 8.8, 1024 x 256 x 256
+//   12.6 / 16.7, 512 x 512 x 1024 39.3 / 44.1, 1024 x 2048 x 512 24.4 / 25.6 (512 tiles:
+//   4096 x 1024 x 256 26 / 18; tiles cut short: 300 x 700 x 2048 94 / 86, at K = 64 8.7 / 9.2)
+//   fp64-folded sums, whose fp32 kernel is slower, up to 64 tiles: the parallel backward at
+//   T16 B16 D256 H32 33.5 / 37.1, T128 B1 D1024 H32 30.7 / 35.3
+//   129 to 256 tiles in two splits: 2048 x 1024 x 512 A^T B 25.6 / 29.1
+bool small_whole(const GemmDesc& d, long s) {
+  const bool whole_m = d.M % 128 == 0 || (d.M > 128 && d.K <= 64 && !d.acc64);
+  if (!vec_rows(d) || !whole_m || d.N % 64 || d.K % 32) return false;
+  const long tiles = tiles_of(d.M, d.N, 128, 64);
+  if (d.acc64) return s == 1 && tiles <= 64;
+  return tiles <= 256 && (s == 1 || (tiles > 128 && d.K < 1024));
 }
 int mid_take(const GemmDesc& d, long max_planes, int* mid) {
   if (!split_products_mode()) return 0;
   const long most = std::max(max_planes, 1L);
-  const bool fold = !(!d.trans_a && d.trans_b);
-  auto fits = [&](long s) { return s > 0 && (!fold || s * kSplitLongKRun >= d.K); };
+  const bool deep = !d.trans_a && d.trans_b && !d.acc64;  // (the fp32 kernel adds all k in one chain)
+  auto fits = [&](long s) { return s > 0 && (deep || s * kSplitLongKRun >= d.K) && !small_whole(d, s); };
   *mid = 1;
   long s = vec_rows(d) ? std::min<long>(gemm_x6_mid_splits(d.M, d.N, d.K, d.trans_a, d.trans_b), most) : 0;
   if (fits(s)) return (int)s;

@@ -24,7 +24,8 @@
 //    stored.  So every shape, aligned or not, runs the one kernel; the slice that holds the
 //    last k is read element by element where a 16-byte load would straddle the end.
 //  * The accumulators restart every 64 k and are added into a second fp32 sum, over at most
-//    kSplitLongKRun k where the product can be split (A^T B, A B); splits are added in fp64.
+//    kSplitLongKRun k for A^T B and A B (A B^T: where a workspace is given and fewer than 256
+//    tiles are there to run); splits are added in fp64.
 //    (Without it the error of A B^T grew past the fp32 kernel's, which split K over waves.)
 //
 // Non-finite operands: a piece product of an infinite value is NaN wherever the other
@@ -265,8 +266,10 @@ int gemm_m6_splits(int M, int N, int K, int trans_a, int trans_b, int lda, int l
   // operands are addressed as raw buffers with 32-bit offsets (a tile's rows may start past the end)
   const size_t a = (size_t)((trans_a ? K : M) + 256) * lda, b = (size_t)((trans_b ? N : K) + 256) * ldb;
   if (a >= ((size_t)1 << 29) || b >= ((size_t)1 << 29)) return 0;
-  if (!trans_a && trans_b) return 1;  // the projection writes C directly
   const long tiles = (long)((M + kMBM - 1) / kMBM) * ((N + kMBN - 1) / kMBN);
+  // A B^T, without the depth bound, is not split once each CU has a workgroup: its planes cost
+  // more than its depth (2100 x 2048 x 512 in one split 43 us, in two 53; 700 x 2600 x 650 36, 34)
+  if (!trans_a && trans_b && tiles >= 256) return 1;
   long s = (768 + tiles - 1) / tiles;  // three workgroups per CU
   s = std::min(s, (long)K / 256);
   s = std::max(s, (long)(K + kSplitLongKRun - 1) / kSplitLongKRun);

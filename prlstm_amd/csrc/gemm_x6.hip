@@ -624,8 +624,11 @@ int x6_pick_splits(long tiles, int M, int N, int K, double us_k, double us_k2, l
 
 int gemm_x6_mid_splits(int M, int N, int K, int trans_a, int trans_b) {
   if ((trans_a && trans_b) || !x6_mid(M, N, K)) return 0;
-  if (!trans_a && trans_b) return 1;
-  return x6_pick_splits(x6_tiles<ShapeMid>(M, N), M, N, K, 0.05, 0.077, (K + kSplitLongKRun - 1) / kSplitLongKRun);
+  const int s =
+      x6_pick_splits(x6_tiles<ShapeMid>(M, N), M, N, K, 0.05, 0.077, (K + kSplitLongKRun - 1) / kSplitLongKRun);
+  // A B^T is split this way only with a caller's workspace; more than 32 planes of few tiles
+  // cost the sum more than they save the product (128 x 256 x 8192: 64 planes 40 us, 32 31)
+  return !trans_a && trans_b ? std::min(s, 32) : s;
 }
 
 bool gemm_x6_applies(int M, int N, int K) {

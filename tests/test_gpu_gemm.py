@@ -280,3 +280,35 @@ def test_middle_split_products_non_finite(dev, split_products, M, N, K, ta, tb):
     ok = torch.isfinite(c32)
     scale = (a.double().abs() @ b.double().abs().t())[ok]
     assert bool(((c6 - c32)[ok].abs() <= 4e-6 * K ** 0.5 * scale).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 200, 16384), (128, 256, 8192), (70, 1030, 4100)])
+def test_deep_products_of_few_tiles_use_the_workspace(dev, split_products, M, N, K):
+    """C = A B^T of few tiles and many k is cut along K into the workspace's planes, which are
+    added in fp64: nearer the fp64 product than the one running sum without a workspace."""
+    print(f"deep A B^T M={M} N={N} K={K}", flush=True)
+    g = torch.Generator().manual_seed(K)
+    a, b = torch.rand(M, K, generator=g), torch.rand(N, K, generator=g)
+    ref = a.double() @ b.double().t()
+    cut, whole = (_gemm(a.to(dev), b.to(dev), None, M, N, K, 0, 1, split=s).cpu().double() for s in (True, False))
+    e_cut, e_whole = float((cut - ref).norm() / ref.norm()), float((whole - ref).norm() / ref.norm())
+    print(f"  planes {e_cut:.3e} one sum {e_whole:.3e}")
+    assert e_cut <= 0.6 * e_whole
+
+
+@pytest.mark.parametrize("M,N,K,ta,tb,ws,fp32", [
+    (256, 512, 64, 0, 1, 0, True), (1024, 2048, 512, 0, 1, 0, True), (2100, 128, 64, 0, 1, 0, True),
+    (1024, 1024, 128, 1, 0, 1, True), (1024, 512, 256, 0, 0, 1, True), (2048, 1024, 512, 1, 0, 1, True),
+    (4096, 1024, 256, 0, 1, 0, False), (300, 704, 2048, 0, 1, 0, False), (1024, 512, 512, 1, 0, 1, False),
+    (1024, 2048, 516, 0, 1, 0, False)])
+def test_which_whole_products_stay_on_the_fp32_kernel(dev, split_products, M, N, K, ta, tb, ws, fp32):
+    """Whole tiles of the fp32 kernel on at most one workgroup per CU, in one split, run there
+    with split products on too (the results are the same bits); their neighbours do not."""
+    g = torch.Generator().manual_seed(K)
+    a = torch.randn(*((K, M) if ta else (M, K)), generator=g).to(dev)
+    b = torch.randn(*((N, K) if tb else (K, N)), generator=g).to(dev)
+    out = []
+    for on in (1, 0):
+        _lib.set_split_products(on)
+        out.append(_gemm(a, b, None, M, N, K, ta, tb, split=bool(ws)))
+    assert torch.equal(*out) == fp32
