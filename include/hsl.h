@@ -50,8 +50,9 @@ int hsl_abi_version(void);
 const char* hsl_last_error(void);
 
 /* Recurrent-path selection: 0 = automatic (persistent kernels where the shape
- * fits on chip in up to four launches over the batch, else one launch per time
- * step), 1 = always per-step, 2 = persistent in one launch of a whole width only
+ * fits on chip in up to four launches over the batch and, for several launches or
+ * a padded width, the sequence is long enough to regain their start; else one launch
+ * per time step), 1 = always per-step, 2 = persistent in one launch of a whole width only
  * (H <= 512, or 1024 or 2048 with B <= 32; else HSL_ERR_UNSUPPORTED).  Returns the previous value.
  * Process-wide. */
 int hsl_set_recurrent_path(int mode);

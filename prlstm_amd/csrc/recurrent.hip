@@ -2074,7 +2074,10 @@ struct OneStepArgs {
   int B, D, H;
   int vec;   // rows of x, h0 and both weights are 16-byte aligned
 };
-constexpr int kOneStepRows = 8;  // batch rows up to which the step runs this way
+// Batch rows up to which the step runs this way: a row costs its products, where the other paths
+// cost the same at any B.  us at D = 256, other paths / here: H = 300 B = 1 15.0 / 7.2, B = 8 15.6 /
+// 11.9; H = 1000 36.3 / 9.4, 36.8 / 17.7; H = 2048 36.0 / 16.5, 36.6 / 31.3, so nearly even at 8.
+constexpr int kOneStepRows = 8;
 
 // acc[g][b] += scale_g * (row of gate g) . (row b), over K columns
 template <int BT, bool VEC>
@@ -2295,9 +2298,26 @@ int bwd_resident(int xt, int ws, int* occ) {
 //            B = 192 (6) 10.4, 16.0 / 10.6, 18.8;  B = 256 (8) 13.8, 22.0 / 11.5, 19.9
 //   H = 384: B = 128 (4) 6.5, 9.7 / 7.2, 14.3;  B = 192 (6) 9.7, 14.4 / 8.9, 16.2
 //   H = 256: B = 128 (2) 2.6, 4.0 / 5.8, 10.6;  H = 128: B = 256 (2) 2.2, 3.7 / 5.1, 9.8
+// (The forward breaks even between 4 and 6; the backward would gain a little up to 6 at H > 256,
+// which this one limit leaves out.  H <= 256 is not measured beyond 4.)
 constexpr int kMaxGroupLaunches = 4;
 
-int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
+// Whether T steps are enough for several launches.  Each starts by loading its W_hh registers
+// (4 to 10 us), and the backward ends by adding one dW_hh plane per group; per step they save
+// less the more of them there are.  Time of launches over time per step, D = 64, by T:
+//   forward, 2 launches: 0.66-0.83 at 4 (H = 450, 4-byte loads of W_hh: 1.36 at 2, 0.94 at 4);
+//     3: 0.86-1.11 at 4 (H = 450 1.31), 0.70-0.92 at 8;  4: 1.1-1.7 at 4, 0.91-1.27 at 8,
+//     0.75-1.00 at 16, except H = 512 B = 128: 1.08 at 16, 0.96 at 32
+//   backward, H >= 100, 2 launches: 0.55-0.99 at 4;  3: 0.84-1.22 at 4, 0.65-0.97 at 8;
+//     4: 0.97-1.18 at 8, 0.68-1.00 at 16;  small H, where a launch holds up to 256 groups:
+//     H = 16, 512 groups (2) 1.05 at 16, 0.77 at 32, 1024 (4) 1.19 at 32, 0.92 at 48;
+//     H = 32, 256 groups (2) 0.99 at 12, 512 (4) 1.11 at 32, 0.98 at 48;  H = 64, 256 (4) 1.00 at 16
+bool group_launches_pay(int T, int H, int groups, int launches, bool bwd) {
+  if (!bwd) return T >= (launches == 4 && H > 448 ? 24 : 1 << launches);
+  return T >= std::max(1 << launches, std::min(64, groups * launches / 40));
+}
+
+int plan_persistent(int T, int B, int H, int D, bool bwd, PersistentPlan* pl) {
   *pl = PersistentPlan{};
   const int mode = recurrent_path_mode();
   if (mode == 1) return HSL_OK;
@@ -2348,7 +2368,8 @@ int plan_persistent(int B, int H, int D, bool bwd, PersistentPlan* pl) {
       p.gpl = (p.NG + p.launches - 1) / p.launches;
       p.NGX = (p.gpl + di.num_xcds - 1) / di.num_xcds * di.num_xcds;
       p.grid = p.NGX * p.NW;
-      p.ok = p.launches <= (mode == 2 ? 1 : kMaxGroupLaunches);
+      p.ok = p.launches == 1 ||
+             (mode != 2 && p.launches <= kMaxGroupLaunches && group_launches_pay(T, H, p.NG, p.launches, bwd));
       p.WS = wgrad_form(kq, H, p.launches);
     }
     if (p.ok || fit > 0 || (p.XT < 0 && !p.XP)) break;
@@ -2418,13 +2439,39 @@ int wide_launches(int H) {
   return H < 1408 ? 1 : H < 1792 ? 2 : 4;
 }
 
-int plan_wide(int B, int H, bool bwd, WidePlan* pl) {
+// Whether T steps are enough for the wide kernels.  Each launch loads W_hh into registers (16 or
+// 64 MB of them, 15 to 40 us), which the widths' own sizes at one launch regain in the first
+// step.  Time of the wide kernels over time per step, D = 64, by T:
+//   512 < H <= 1024, one launch: forward 0.95 or less, backward 0.81-1.03 at 1;  two (H % 4 != 0):
+//     forward 0.79-1.12 at 2, 0.72-0.99 at 4, backward 0.91-1.03 at 4, 0.86-0.99 at 6
+//   1024 < H, one launch of at most 16 rows (B) or more: forward 1.04 or less at 1 (H < 1300 with
+//     B > 16: 1.10 at 1, 0.98 at 8);  backward B <= 16: H = 1100 1.12 at 4, 1.00 at 6, 1500 1.02
+//     at 3, 0.96 at 4, 1700 1.05 at 2, 0.96 at 3, 2000 1.05 at 1, 0.94 at 2;  B > 16: H = 1100 1.05 at 12, 1.00
+//     at 16, 1300 1.03 at 8, 0.96 at 12, 1500 1.06 at 4, 0.98 at 6, 1800 1.04 at 2, 0.95 at 4, 2000 0.99 at 2
+//   two to four launches: forward H = 1500 1.03 at 8, 0.98 at 12, 1700 to 2048 1.07 at 4,
+//     0.85-0.99 at 8;  backward H = 1500 1.02 at 12, 0.96 at 16, 1700 to 2000 two and three 0.82-0.99
+//     at 8, four 1.04 at 12, 0.98 at 16;  H = 2048 two 0.89 at 1, three 0.96 at 2, four 0.99 at 4
+bool wide_pays(int T, int B, int H, int launches, bool bwd) {
+  if (H <= 1024) return launches == 1 || T >= (bwd ? 6 : 4);
+  if (launches == 1) {
+    if (H == 2048) return true;
+    if (!bwd) return B <= 16 || H >= 1300 || T >= 8;
+    if (B <= 16) return T >= (H < 1350 ? 6 : H < 1600 ? 4 : H < 1900 ? 3 : 2);
+    return T >= (H < 1250 ? 16 : H < 1350 ? 12 : H < 1600 ? 8 : H < 1900 ? 4 : 2);
+  }
+  if (!bwd) return T >= (H < 1600 ? 12 : 8);
+  if (H == 2048) return T >= (launches == 4 ? 4 : launches == 3 ? 2 : 1);
+  return T >= (H < 1600 || launches == 4 ? 16 : 8);
+}
+
+int plan_wide(int T, int B, int H, bool bwd, WidePlan* pl) {
   *pl = WidePlan{};
   const int mode = recurrent_path_mode();
   const int U = wide_u(H);
   if (mode == 1 || B < 1 || U == 0) return HSL_OK;
   const int launches = (B + 31) / 32;
-  if (launches > wide_launches(H) || (mode == 2 && (launches > 1 || H != 32 * U))) return HSL_OK;
+  if (mode == 2 ? launches > 1 || H != 32 * U : launches > wide_launches(H) || !wide_pays(T, B, H, launches, bwd))
+    return HSL_OK;
   DeviceInfo di;
   HSL_CHECK(device_info(&di));
   if (di.num_xcds != kWideXcds || di.num_cus < kWideWgs) return HSL_OK;
@@ -2778,8 +2825,8 @@ int rec_fwd(const float* x, const float* h0, const float* c0, const float* w_ih,
   }
   PersistentPlan pl;
   WidePlan wp;
-  if (!per_step) HSL_CHECK(plan_persistent(B, H, D, false, &pl));
-  if (!per_step && !pl.ok) HSL_CHECK(plan_wide(B, H, false, &wp));
+  if (!per_step) HSL_CHECK(plan_persistent(T, B, H, D, false, &pl));
+  if (!per_step && !pl.ok) HSL_CHECK(plan_wide(T, B, H, false, &wp));
   if (recurrent_path_mode() == 2 && !pl.ok && !wp.ok)
     return fail(HSL_ERR_UNSUPPORTED, "persistent path does not fit (B=%d H=%d)", B, H);
   const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
@@ -2917,7 +2964,7 @@ size_t hsl_rec_fwd_ws_bytes(int T, int B, int D, int H) {
   WidePlan wp;
   if (one_step(T, B, D))
     nd.xch = nd.gih = nd.step = nd.wide = false;
-  else if (B > 0 && H > 0 && plan_persistent(B, H, D, false, &pl) == HSL_OK && plan_wide(B, H, false, &wp) == HSL_OK)
+  else if (B > 0 && H > 0 && plan_persistent(T, B, H, D, false, &pl) == HSL_OK && plan_wide(T, B, H, false, &wp) == HSL_OK)
     nd = fwd_needs(pl, wp, true);
   return carve_fwd(nullptr, 0, T, B, H, nd, &w);
 }
@@ -2935,9 +2982,9 @@ int hsl_rec_fwd_noalloc(const float* x, const float* h0, const float* c0, const 
   HSL_CHECK(check_dims(T, B, D, H));
   if (B == 0 || H == 0) return HSL_OK;
   PersistentPlan pl;
-  HSL_CHECK(plan_persistent(B, H, D, false, &pl));
+  HSL_CHECK(plan_persistent(T, B, H, D, false, &pl));
   WidePlan wp;
-  if (!pl.ok) HSL_CHECK(plan_wide(B, H, false, &wp));
+  if (!pl.ok) HSL_CHECK(plan_wide(T, B, H, false, &wp));
   const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
   if (pl.XP && !x_aligned) pl.XP = false;
   FwdWs w;
@@ -2972,7 +3019,7 @@ size_t hsl_rec_bwd_ws_bytes_for(int T, int B, int D, int H, int with_dx) {
   BwdNeeds nd;  // every part when the path cannot be planned (no device)
   PersistentPlan pl;
   WidePlan wp;
-  if (B > 0 && H > 0 && plan_persistent(B, H, D, true, &pl) == HSL_OK && plan_wide(B, H, true, &wp) == HSL_OK)
+  if (B > 0 && H > 0 && plan_persistent(T, B, H, D, true, &pl) == HSL_OK && plan_wide(T, B, H, true, &wp) == HSL_OK)
     nd = bwd_needs(pl, wp, with_dx != 0);
   return carve_bwd(nullptr, 0, T, B, D, H, nd, &w);
 }
@@ -2992,8 +3039,8 @@ int hsl_rec_bwd(const float* dout, const float* dh_n, const float* dc_n, const f
     return fail(HSL_ERR_ARG, "hsl_rec_bwd: null pointer");
   PersistentPlan pl;
   WidePlan wp;
-  if (T > 0 && B > 0 && H > 0) HSL_CHECK(plan_persistent(B, H, D, true, &pl));
-  if (T > 0 && B > 0 && H > 0 && !pl.ok) HSL_CHECK(plan_wide(B, H, true, &wp));
+  if (T > 0 && B > 0 && H > 0) HSL_CHECK(plan_persistent(T, B, H, D, true, &pl));
+  if (T > 0 && B > 0 && H > 0 && !pl.ok) HSL_CHECK(plan_wide(T, B, H, true, &wp));
   if (T > 0 && B > 0 && H > 0 && recurrent_path_mode() == 2 && !pl.ok && !wp.ok)
     return fail(HSL_ERR_UNSUPPORTED, "persistent path does not fit (B=%d H=%d)", B, H);
   BwdWs w;

@@ -164,9 +164,9 @@ def test_forward_quarters_of_96(dev, H, B, D, scope):
 
 
 @pytest.mark.parametrize("T,B,D,H", [(9, 33, 20, 512),    # 9 groups: launches of 5 and 4
-                                     (3, 128, 16, 512),   # the most launches: 4 of 8 groups
+                                     (24, 128, 16, 512),  # the most launches: 4 of 8 groups
                                      (9, 66, 270, 300),   # D > 256: separate dW_ih, dgates of both launches
-                                     (2, 261, 12, 20)])   # 66 groups of two workgroups, a last group of one row
+                                     (4, 261, 12, 20)])   # 66 groups of two workgroups, a last group of one row
 def test_batch_over_several_launches(dev, T, B, D, H):
     """A batch of more groups than the chip holds at once runs as several launches of the
     persistent kernels, each over its own groups of the same buffers (path 2); a fifth launch
@@ -183,6 +183,21 @@ def test_one_step_of_few_rows(dev, B, D, H, with_hx):
     check(1, B, D, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=with_hx, fwd_path=1)
     if H == 300:
         check(1, B + 1, D, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=with_hx, fwd_path=2)
+
+
+@pytest.mark.parametrize("T,B,H,fwd,bwd", [
+    (3, 40, 260, 1, 1), (4, 40, 260, 2, 2), (7, 270, 128, 1, 1), (8, 270, 128, 2, 2),     # 2 and 3 launches
+    (15, 100, 300, 1, 1), (16, 100, 300, 2, 2), (16, 100, 450, 1, 2),                     # 4 launches
+    (6, 576, 32, 2, 1), (8, 576, 32, 2, 2),                                               # 144 groups
+    (1, 9, 520, 3, 3), (4, 33, 650, 3, 1), (6, 33, 650, 3, 3),                            # width 1024
+    (1, 9, 1100, 3, 1), (6, 9, 1100, 3, 3), (7, 17, 1100, 1, 1), (8, 17, 1100, 3, 1),     # width 2048
+    (3, 9, 1500, 3, 1), (1, 9, 2000, 3, 1), (2, 17, 2000, 3, 3), (1, 40, 2048, 1, 3), (8, 40, 1800, 3, 3)])
+def test_short_sequences_take_the_faster_path(dev, T, B, H, fwd, bwd):
+    """Several launches, and the wide kernels below their own widths, have to load W_hh first:
+    sequences of a few steps run per step, forward and backward each by its own line (3 is the
+    wide kernels, 2 the launches over the batch)."""
+    check(T, B, 16, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=True, fwd_path=fwd)
+    assert prlstm_amd.last_recurrent_path() == bwd
 
 
 def test_weight_gradient_of_several_launches_is_as_accurate_as_per_step(dev):
@@ -278,8 +293,8 @@ def test_wide_short_sequences(dev, T, B, H):
 
 
 @pytest.mark.parametrize("T,B,H", [(7, 5, 513), (6, 20, 650), (9, 32, 771), (5, 18, 1023),    # width 1024
-                                   (6, 3, 1025), (5, 32, 1500), (4, 17, 2047),               # width 2048
-                                   (6, 33, 650), (3, 50, 1500), (2, 70, 1800)])              # two and three launches
+                                   (6, 3, 1025), (8, 32, 1500), (4, 17, 2047),               # width 2048
+                                   (6, 33, 650), (16, 50, 1500), (8, 70, 1800)])             # two and three launches
 def test_wide_kernels_padded_width_and_batch_launches(dev, T, B, H):
     """Hidden sizes between the wide kernels' own widths run on the next width, whose units past
     H keep every hand-off's order but read and store nothing (H a multiple of 4 or not: 16- or
