@@ -60,6 +60,23 @@ int hsl_set_recurrent_path(int mode);
  * workgroup (default 2,000,000).  On expiry the kernel stops and raises the
  * device error flag instead of waiting forever.  Returns the previous value. */
 long long hsl_set_spin_timeout_us(long long us);
+/* The persistent kernels' workgroups wait for each other, so all of a launch must be
+ * resident at once, one per CU.  Calls of one process on several streams are ordered
+ * by the library where their launches would not fit side by side (the later stream
+ * waits for the earlier one's call).  The replay of a graph that captured hsl_rec_fwd
+ * or hsl_rec_bwd is ordered with them when it stands between the two calls below, on
+ * the thread and stream that launch it (prlstm_amd.graph does so), with the workgroups
+ * of its largest launch; the thread holds the library's launch lock between them.
+ * hsl_launched_workgroups gives the workgroups of the largest persistent launch of
+ * this process since it was last called with clear != 0 (0: none, as in the per-step
+ * path and the scans, which need no order).  Not ordered, and for the caller to
+ * keep apart: other replays, other processes on the device, and kernels of other
+ * libraries that hold CUs while they wait (a collective whose peers come late).  A
+ * launch that waits for its workgroups longer than the spin limit fails as described
+ * there.  A stream is to be destroyed only when its calls have ended. */
+int hsl_launched_workgroups(int clear);
+int hsl_replay_begin(int workgroups, void* stream);
+int hsl_replay_end(void);
 /* Hand-off between the workgroups of a persistent kernel: 0 = automatic (stores
  * that stay in the XCD's L2 when the launch verifies that every workgroup of a
  * batch group runs on one XCD, device-scope stores otherwise), 1 = always

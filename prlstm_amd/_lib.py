@@ -27,6 +27,9 @@ SIGNATURES = {
     "hsl_set_spin_timeout_us": (ctypes.c_longlong, [ctypes.c_longlong]),
     "hsl_last_recurrent_path": (_I, []),
     "hsl_last_backward_fused": (_I, []),
+    "hsl_launched_workgroups": (_I, [_I]),
+    "hsl_replay_begin": (_I, [_I, _P]),
+    "hsl_replay_end": (_I, []),
     "hsl_set_exchange_scope": (_I, [_I]),
     "hsl_set_split_products": (_I, [_I]),
     "hsl_poll_error": (_I, [_P, _P, _P]),

@@ -54,6 +54,23 @@ struct TimingSuppress {
   TimingSuppress(const TimingSuppress&) = delete;
   TimingSuppress& operator=(const TimingSuppress&) = delete;
 };
+// The launches of the persistent kernels on different streams, ordered where they could not all
+// be resident.  Their workgroups wait for each other, one per CU: two launches that each hold
+// part of the CUs would wait until the spin limit.  An object lives from before the first to
+// after the last launch of one call: it makes `stream` wait for the launches that other streams
+// of this process hold when together they exceed the device's CUs, and notes the call's own.
+// Nothing is ordered inside a capture (the graph's replays are what runs, see hsl_replay_begin).
+class LaunchOrder {
+ public:
+  LaunchOrder(int workgroups, hipStream_t stream);
+  ~LaunchOrder();
+  LaunchOrder(const LaunchOrder&) = delete;
+  LaunchOrder& operator=(const LaunchOrder&) = delete;
+
+ private:
+  int device_ = -1;  // -1: not ordered (no device)
+  hipStream_t stream_;
+};
 long long spin_timeout_ticks();   // in wall_clock64 ticks (100 MHz)
 void note_recurrent_path(int path);
 void note_backward_fused(int fused);  // 0, 1 (dW_hh) or 2 (dW_hh and dW_ih)

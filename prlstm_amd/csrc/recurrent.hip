@@ -25,6 +25,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <optional>
 #include <cstdlib>
 #include <type_traits>
 
@@ -2837,6 +2838,8 @@ int rec_fwd(const float* x, const float* h0, const float* c0, const float* w_ih,
     return fail(HSL_ERR_ARG, "hsl_rec_fwd: workspace %zu bytes, need %zu%s", ws_bytes, need,
                 pl.ok && !x_aligned ? " (x is not 16-byte aligned, so the input-gate buffer is needed)" : "");
 
+  std::optional<LaunchOrder> order;
+  if (T > 0 && (pl.ok || wp.ok)) order.emplace(pl.ok ? pl.grid : kWideWgs, s);
   if (pl.ok && T > 0)
     HSL_CHECK(prepare_persistent(w.err, w.xbuf, w.xfloats, w.hello, w.hwords, s));
   else if (wp.ok && T > 0)
@@ -3073,6 +3076,8 @@ int hsl_rec_bwd(const float* dout, const float* dh_n, const float* dc_n, const f
     nsplit = (T + wts - 1) / wts * pl.NG;
     wpx = wph + (size_t)nsplit * 4 * H * H;
   }
+  std::optional<LaunchOrder> order;
+  if (pl.ok || wp.ok) order.emplace(pl.ok ? pl.grid : kWideWgs, s);
   if (pl.ok)
     HSL_CHECK(prepare_persistent(w.err, w.pbuf, w.pfloats, w.hello, w.hwords, s));
   else if (wp.ok)
@@ -3165,6 +3170,7 @@ int hsl_rec_bwd(const float* dout, const float* dh_n, const float* dc_n, const f
     note_recurrent_path(1);
   }
 
+  order.reset();  // the persistent launches are queued
   // dW_hh_s = dg^T h_prev (staged partials), then dW_hh = a dW_hh_s and the da row sums.
   // A one-split product does the second part in its own epilogue (dot_parts > 0).
   int splits = nsplit, dot_parts = 0;

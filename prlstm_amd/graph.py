@@ -17,7 +17,25 @@ parameters' ``.grad`` point at the gradients of the mode just replayed, or are
 parallel mode), exactly as an eager step leaves them.
 """
 
+import contextlib
+import threading
+
 import torch
+
+from . import _lib
+
+_capture_lock = threading.Lock()  # one capture at a time counts the library's launches
+
+
+@contextlib.contextmanager
+def _replay_order(workgroups, device):
+    """Orders what is replayed inside with the persistent launches of this process's other
+    streams, as the library orders eager calls: `workgroups` of a launch wait for each other."""
+    _lib.call("hsl_replay_begin", workgroups, _lib.stream_of(device))
+    try:
+        yield
+    finally:
+        _lib.call("hsl_replay_end")
 
 
 class GraphedTrainStep:
@@ -58,15 +76,18 @@ class GraphedTrainStep:
         torch.cuda.current_stream().wait_stream(side)
         m.zero_grad(set_to_none=True)
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            out, (h_n, c_n) = m(self.static_x, self.hx)
-            torch.autograd.backward([out], [self.grad_out])
+        with _capture_lock:
+            _lib.load().hsl_launched_workgroups(1)
+            with torch.cuda.graph(graph):
+                out, (h_n, c_n) = m(self.static_x, self.hx)
+                torch.autograd.backward([out], [self.grad_out])
+            workgroups = _lib.load().hsl_launched_workgroups(0)
         grads = {n: p.grad for n, p in m.named_parameters()}
         # Only detached views of the static outputs are kept (same memory): the captured
         # autograd graph, and with it the parameters' AccumulateGrad nodes created on the
         # capture stream, is released, so later eager steps on another stream build their
         # own nodes instead of reusing those (a stream mismatch torch warns about).
-        self._graphs[mode] = (graph, out.detach(), h_n.detach(), c_n.detach(), grads)
+        self._graphs[mode] = (graph, out.detach(), h_n.detach(), c_n.detach(), grads, workgroups)
         del out, h_n, c_n
 
     @property
@@ -82,10 +103,14 @@ class GraphedTrainStep:
         mode = bool(self.module.parallel)
         if mode not in self._graphs:
             self._capture(mode)
-        graph, out, h_n, c_n, grads = self._graphs[mode]
+        graph, out, h_n, c_n, grads, workgroups = self._graphs[mode]
         if x is not None:
             self.static_x.copy_(x)
-        graph.replay()
+        if workgroups:
+            with _replay_order(workgroups, self.static_x.device):
+                graph.replay()
+        else:
+            graph.replay()
         for n, p in self.module.named_parameters():
             p.grad = grads[n]
         self.static_out, self.static_h_n, self.static_c_n = out, h_n, c_n

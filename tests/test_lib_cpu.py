@@ -81,6 +81,7 @@ def test_argument_errors_are_reported_without_a_gpu():
     assert rc == 1 and b"leading dimension" in lib.hsl_last_error()
     with pytest.raises(RuntimeError, match="hsl_rec_fwd failed"):
         _lib.call("hsl_rec_fwd", *([None] * 12), None, 0, 1, 1, 1, 1, None)
+    assert lib.hsl_replay_end() == 1 and b"no hsl_replay_begin" in lib.hsl_last_error()
     # the fp64 entry points refuse null operands before any launch
     for name, args in (
             ("hsl_rec_fwd_f64", [None] * 13 + [0, 4, 2, 3, 5, None]),
