@@ -78,20 +78,27 @@ def split_products():
     _lib.set_split_products(prev)
 
 
-def _both(A, B, bias, M, N, K, lda=None, ldb=None, ta=0, tb=1):
+SENTINEL = -12345.5
+
+
+def _both(A, B, bias, M, N, K, lda=None, ldb=None, ta=0, tb=1, ldc=None):
     """C = op(A) op(B) (+bias) by the split-bf16 kernel and by the fp32 MFMA kernel
-    (A B^T by default; ta=1, tb=0 for A^T B, with the workspace hsl_gemm_ws_bytes asks)."""
+    (A B^T by default; ta=1, tb=0 for A^T B, with the workspace hsl_gemm_ws_bytes asks).
+    C has a row before it, one after it and ldc - N columns beside it that must stay as they are."""
     dev = A.device
     out = []
     nbytes = _lib.load().hsl_gemm_ws_bytes(M, N, K)
     ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
     for on in (1, 0):
         _lib.set_split_products(on)
-        C = torch.empty(M, N, device=dev)
+        buf = torch.full((M + 2, ldc or N), SENTINEL, device=dev)
+        C = buf[1:M + 1]
         P = _lib.ptr
-        _lib.call("hsl_gemm_f32", P(A), P(B), P(bias), P(C), M, N, K, lda or A.shape[1], ldb or B.shape[1], N,
+        _lib.call("hsl_gemm_f32", P(A), P(B), P(bias), P(C), M, N, K, lda or A.shape[1], ldb or B.shape[1], ldc or N,
                   ta, tb, P(ws), nbytes, _lib.stream_of(dev))
-        out.append(C.cpu().double())
+        out.append(C[:, :N].cpu().double())
+        C[:, :N] = SENTINEL
+        assert bool((buf == SENTINEL).all())
     _lib.set_split_products(1)
     return out
 
@@ -244,13 +251,14 @@ LAYOUTS = [(0, 0), (0, 1), (1, 0)]
 def test_middle_split_products(dev, split_products, M, N, K, ta, tb, pad):
     """Middle-sized and ragged products on split pieces, with and without 16-byte aligned rows:
     the fp32 bound against fp64, an rms error not above the fp32 kernel's (5% for the sampling
-    noise of the rms), and nothing written past the rows of C."""
+    noise of the rms; the fp64-folded sums of the backward are compared below), and nothing
+    written beside C, whose rows are also longer than N here."""
     print(f"middle split products M={M} N={N} K={K} ta={ta} tb={tb} pad={pad}", flush=True)
     g = torch.Generator().manual_seed(M + N + K)
     a = torch.randn(*((K, M + pad) if ta else (M, K + pad)), generator=g)
     b = torch.randn(*((N, K + pad) if tb else (K, N + pad)), generator=g) * 0.1
     bias = torch.randn(N, generator=g)
-    c6, c32 = _both(a.to(dev), b.to(dev), bias.to(dev), M, N, K, ta=ta, tb=tb)
+    c6, c32 = _both(a.to(dev), b.to(dev), bias.to(dev), M, N, K, ta=ta, tb=tb, ldc=N + 5 * pad)
     assert not torch.equal(c6, c32)  # two different kernels ran
     av = (a[:, :M].t() if ta else a[:, :K]).double()
     bv = (b[:, :K].t() if tb else b[:, :N]).double()
@@ -312,3 +320,38 @@ def test_which_whole_products_stay_on_the_fp32_kernel(dev, split_products, M, N,
         _lib.set_split_products(on)
         out.append(_gemm(a, b, None, M, N, K, ta, tb, split=bool(ws)))
     assert torch.equal(*out) == fp32
+
+
+@pytest.mark.parametrize("mean", [0.0, 0.5, 2.0])
+@pytest.mark.parametrize("T,B,D,H", [(256, 8, 128, 512),    # K = 2048 either way, whole tiles
+                                     (256, 7, 100, 333),    # ragged
+                                     (35, 20, 650, 650),    # dx over K = 2600
+                                     (128, 32, 256, 256)])  # dW_ih over K = 4096
+def test_middle_gradients_as_accurate_as_fp64_folded_sums(dev, split_products, T, B, D, H, mean):
+    """The weight gradient and dx products of the backward: with split products off their fp32
+    kernel folds every 128 k into fp64.  The split pieces' fp32 sums are no further from the
+    64-bit products of the same operands, of zero mean and not (5% for the noise of the rms)."""
+    print(f"gradients T={T} B={B} D={D} H={H} mean={mean}", flush=True)
+    lib, P, s = _lib.load(), _lib.ptr, _lib.stream_of(dev)
+    g = torch.Generator(device=dev).manual_seed(T + H)
+    rand = lambda *shape: torch.randn(*shape, device=dev, generator=g)  # noqa: E731
+    gates, x, w, dout, c0 = rand(T, B, 4 * H), rand(T, B, D) + mean, rand(4 * H, D) + mean, rand(T, B, H) + mean, \
+        rand(B, H).abs()
+    out, ck = torch.empty(T, B, H, device=dev), torch.empty(lib.hsl_scan_ck_rows(T), B, H, device=dev)
+    _lib.call("hsl_scan_fwd", P(gates), P(c0), 1e-6, P(out), P(ck), T, B, H, s)
+    dg = torch.empty_like(gates)  # (T is short enough that the backward's scan is this one, uncut)
+    _lib.call("hsl_scan_bwd", P(gates), P(c0), P(ck), P(dout), None, None, 1e-6, P(dg), None, None, T, B, H, s)
+    dg, x2 = dg.double().view(T * B, 4 * H), x.double().view(T * B, D)
+    want = {"dw": dg.t() @ x2, "dx": dg @ w.double()}
+    err = {}
+    for on in (1, 0):
+        _lib.set_split_products(on)
+        n = lib.hsl_par_bwd_ws_bytes(T, B, D, H)
+        ws = torch.empty(n, dtype=torch.uint8, device=dev)
+        got = {"dw": torch.empty(4 * H, D, device=dev), "dx": torch.empty(T * B, D, device=dev)}
+        _lib.call("hsl_par_bwd", P(dout), None, None, P(x), P(c0), P(gates), P(ck), P(w), 1e-6, P(got["dx"]),
+                  P(got["dw"]), P(torch.empty(4 * H, device=dev)), None, P(ws), n, T, B, D, H, s)
+        err[on] = {k: float((got[k].double() - v).norm() / v.norm()) for k, v in want.items()}
+    print(err)
+    for k in want:
+        assert err[1][k] <= 1.05 * err[0][k] <= 1e-6, k
