@@ -457,7 +457,7 @@ __device__ __forceinline__ void x6_tile(const X6Args& g, int m0, int n0, unsigne
 #pragma unroll
         for (int j = 0; j < S::FN; ++j) {
           f16v& res = S::FOLD ? tot[S::FOLD ? i : 0][S::FOLD ? j : 0] : acc[i][j];
-          const int m = min(m0 + wm * S::TM + 32 * i + r32, g.M - 1), n = min(n0 + wn * S::TN + 32 * j + r32, g.N - 1);
+          const int m = m0 + wm * S::TM + 32 * i + r32, n = n0 + wn * S::TN + 32 * j + r32;  // whole tiles
           f16v sum = f16v{}, run = f16v{};
           for (int k = kbeg; k < kend; k += 2) {
             const int kk = k + half;
@@ -571,16 +571,25 @@ __global__ __launch_bounds__(kThreads, S::BM == 128 ? 4 : 1) void gemm_x6_kernel
   x6_tile<S, FULL, AKC, BKC, BP>(g, tm * S::BM, tn * S::BN, x6_smem);
 }
 
+// The 128 x 128 tiles and the tiles with a bf16 operand only take whole tiles of aligned rows
+// (gemm_x6_mid_splits, gemm_x6_full): other products of their sizes run on gemm_m6.hip.
+template <class S, int BP>
+constexpr bool kMasked = S::BM == 256 && BP == 3;
+
 template <class S, bool AKC, bool BKC, int BP = 3>
-void x6_launch(X6Args g, bool vec, int splits, hipStream_t s) {
+int x6_launch(X6Args g, bool vec, int splits, hipStream_t s) {
   g.tiles_m = (g.M + S::BM - 1) / S::BM;
   g.tiles_n = (g.N + S::BN - 1) / S::BN;
   const bool full = vec && g.M % S::BM == 0 && g.N % S::BN == 0 && g.K % kBK == 0 && g.kps % kBK == 0;
   const dim3 grid(g.tiles_m * g.tiles_n, 1, splits);
   if (full)
     hipLaunchKernelGGL((gemm_x6_kernel<S, true, AKC, BKC, BP>), grid, dim3(kThreads), S::LDS, s, g);
-  else
+  else if constexpr (kMasked<S, BP>)
     hipLaunchKernelGGL((gemm_x6_kernel<S, false, AKC, BKC, BP>), grid, dim3(kThreads), S::LDS, s, g);
+  else
+    return fail(HSL_ERR_ARG, "gemm_x6: %d x %d x %d is not whole tiles of aligned rows", g.M, g.N, g.K);
+  HSL_HIP(hipGetLastError());
+  return HSL_OK;
 }
 
 }  // namespace
@@ -681,8 +690,7 @@ int gemm_x6_wgrad_fin(const float* A, const float* B, float* C, const float* a_g
   g.rs_rows = group_rows;
   g.dotw = W;
   g.dotp = dotp;
-  x6_launch<S, false, false>(g, true, 1, s);
-  HSL_HIP(hipGetLastError());
+  HSL_CHECK((x6_launch<S, false, false>(g, true, 1, s)));
   *parts = (int)(n / (M / group_rows));
   return HSL_OK;
 }
@@ -713,26 +721,16 @@ int gemm_x6_run(const float* A, const void* B, const float* bias, float* C, floa
   if (used) *used = n;
   const bool vec = aligned16(A) && aligned16(B) && lda % 4 == 0 && ldb % 4 == 0;
   g.out_vec = aligned16(g.out) && (partial ? N % 4 == 0 : ldc % 4 == 0) && (g.bias == nullptr || aligned16(g.bias));
-  if (mid && !trans_a && trans_b)
-    x6_launch<ShapeMid, true, true>(g, vec, n, s);
-  else if (mid && trans_a)
-    x6_launch<ShapeMid, false, false>(g, vec, n, s);
-  else if (mid)
-    x6_launch<ShapeMid, true, false>(g, vec, n, s);
-  else if (b_bf16 && trans_a)
-    x6_launch<ShapeWgrad, false, false, 1>(g, vec, n, s);  // dgates^T x with a bf16 x
-  else if (b_bf16)
-    x6_launch<ShapeWgrad, true, false, 1>(g, vec, n, s);  // dgates W_ih with a bf16 W_ih
-  else if (!trans_a && trans_b && x6_tiles<ShapeProj>(M, N) >= 256)
-    x6_launch<ShapeProj, true, true>(g, vec, n, s);  // x W^T: both operands k-contiguous
-  else if (!trans_a && trans_b)
-    x6_launch<ShapeWgrad, true, true>(g, vec, n, s);  // the same on 256 x 128 tiles (fewer than 256 of 256 x 256)
-  else if (trans_a)
-    x6_launch<ShapeWgrad, false, false>(g, vec, n, s);  // A^T B: both row-contiguous
-  else
-    x6_launch<ShapeWgrad, true, false>(g, vec, n, s);  // A B (dx = dgates W_ih): B row-contiguous
-  HSL_HIP(hipGetLastError());
-  return HSL_OK;
+  if (mid && !trans_a && trans_b) return x6_launch<ShapeMid, true, true>(g, vec, n, s);
+  if (mid && trans_a) return x6_launch<ShapeMid, false, false>(g, vec, n, s);
+  if (mid) return x6_launch<ShapeMid, true, false>(g, vec, n, s);
+  if (b_bf16 && trans_a) return x6_launch<ShapeWgrad, false, false, 1>(g, vec, n, s);  // dgates^T x with a bf16 x
+  if (b_bf16) return x6_launch<ShapeWgrad, true, false, 1>(g, vec, n, s);              // dgates W_ih with a bf16 W_ih
+  // x W^T, both operands k-contiguous: 256 x 256 tiles, or 256 x 128 where those are fewer than 256
+  if (!trans_a && trans_b && x6_tiles<ShapeProj>(M, N) >= 256) return x6_launch<ShapeProj, true, true>(g, vec, n, s);
+  if (!trans_a && trans_b) return x6_launch<ShapeWgrad, true, true>(g, vec, n, s);
+  if (trans_a) return x6_launch<ShapeWgrad, false, false>(g, vec, n, s);  // A^T B: both row-contiguous
+  return x6_launch<ShapeWgrad, true, false>(g, vec, n, s);                // A B (dx = dgates W_ih): B row-contiguous
 }
 
 }  // namespace hsl
