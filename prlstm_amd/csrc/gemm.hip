@@ -233,7 +233,13 @@ bool vec_rows(const GemmDesc& d) {
 //   fp64-folded sums, whose fp32 kernel is slower, up to 64 tiles: the parallel backward at
 //   T16 B16 D256 H32 33.5 / 37.1, T128 B1 D1024 H32 30.7 / 35.3
 //   129 to 256 tiles in two splits: 2048 x 1024 x 512 A^T B 25.6 / 29.1
-bool small_whole(const GemmDesc& d, long s) {
+//   fewer than 64 columns, where the fp32 kernel is that of 32 x 32 tiles with K cut over its waves:
+//   A B^T 1000 x 60 x 300 7 / 18, with planes 1000 x 60 x 16384 38 / 44, 2048 x 60 x 16384 65 / 53,
+//   without 2048 x 60 x 4096 61 / 170; fp64-folded, the parallel backward at D = 33 to 63 (M K =
+//   4 H T B for both products) 1.1 to 1.5 times as long on split pieces at M K = 1.3e5 to 3e6, as
+//   long at 6e6, 0.8 times at 1.7e7
+bool stays_fp32(const GemmDesc& d, long s) {
+  if (d.N < 64) return d.acc64 ? (double)d.M * d.K < 6.5e6 : s < 2 || (double)d.M * d.K < 2e7;
   const bool whole_m = d.M % 128 == 0 || (d.M > 128 && d.K <= 64 && !d.acc64);
   if (!vec_rows(d) || !whole_m || d.N % 64 || d.K % 32) return false;
   const long tiles = tiles_of(d.M, d.N, 128, 64);
@@ -244,7 +250,7 @@ int mid_take(const GemmDesc& d, long max_planes, int* mid) {
   if (!split_products_mode()) return 0;
   const long most = std::max(max_planes, 1L);
   const bool deep = !d.trans_a && d.trans_b && !d.acc64;  // (the fp32 kernel adds all k in one chain)
-  auto fits = [&](long s) { return s > 0 && (deep || s * kSplitLongKRun >= d.K) && !small_whole(d, s); };
+  auto fits = [&](long s) { return s > 0 && (deep || s * kSplitLongKRun >= d.K) && !stays_fp32(d, s); };
   *mid = 1;
   long s = vec_rows(d) ? std::min<long>(gemm_x6_mid_splits(d.M, d.N, d.K, d.trans_a, d.trans_b), most) : 0;
   if (fits(s)) return (int)s;
