@@ -91,7 +91,7 @@ int hsl_set_exchange_scope(int mode);
  *    gradients and dx (_torch.py:157-162), as fp32 runs of 64 k folded into a second
  *    fp32 sum, split along K into planes of at most 2048 k added in fp64 (workspace
  *    permitting; otherwise the fp32 kernel runs);
- *  - smaller ones with M >= 64, N > 32, K >= 64 and at least 6e6 multiply-adds, and those
+ *  - smaller ones with M, N, K >= 64 and at least 6e6 multiply-adds, and those
  *    whose sizes or alignment the large tiles do not fit; non-finite operands keep the fp32
  *    instruction's results there (such a tile is computed again with it);
  *  - the products the persistent recurrent kernels fuse (H <= 512): the forward's input

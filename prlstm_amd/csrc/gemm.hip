@@ -225,26 +225,20 @@ bool vec_rows(const GemmDesc& d) {
   return aligned16(d.A) && aligned16(d.B) && d.lda % 4 == 0 && d.ldb % 4 == 0;
 }
 // Products that stay on the fp32 kernel (gemm3_core.h): whole tiles of it, few enough that a
-// CU has one workgroup or none, where its shorter slices (no split, no fold) are the lower
-// latency.  us, fp32 kernel / split pieces:
-//   one split, up to 256 tiles of 128 x 64: A B^T 256 x 512 x 64 5.8 / 8.8, 1024 x 256 x 256
-//   12.6 / 16.7, 512 x 512 x 1024 39.3 / 44.1, 1024 x 2048 x 512 24.4 / 25.6 (512 tiles:
-//   4096 x 1024 x 256 26 / 18; tiles cut short: 300 x 700 x 2048 94 / 86, at K = 64 8.7 / 9.2)
-//   fp64-folded sums, whose fp32 kernel is slower, up to 64 tiles: the parallel backward at
-//   T16 B16 D256 H32 33.5 / 37.1, T128 B1 D1024 H32 30.7 / 35.3
-//   129 to 256 tiles in two splits: 2048 x 1024 x 512 A^T B 25.6 / 29.1
-//   fewer than 64 columns, where the fp32 kernel is that of 32 x 32 tiles with K cut over its waves:
-//   A B^T 1000 x 60 x 300 7 / 18, with planes 1000 x 60 x 16384 38 / 44, 2048 x 60 x 16384 65 / 53,
-//   without 2048 x 60 x 4096 61 / 170; fp64-folded, the parallel backward at D = 33 to 63 (M K =
-//   4 H T B for both products) 1.1 to 1.5 times as long on split pieces at M K = 1.3e5 to 3e6, as
-//   long at 6e6, 0.8 times at 1.7e7
+// CU has one workgroup or none, and few k, where its shorter slices (no split, no fold) are the
+// lower latency and its longer sums still cost little.  us and relative error, fp32 kernel / split
+// pieces, A B^T of up to 256 tiles of 128 x 64:
+//   256 x 512 x 64 5.8 / 8.8, 1.5e-7 / 1.3e-7;  1024 x 256 x 128 8.0 / 11.4, 2.0e-7 / 1.4e-7;
+//   512 x 512 x 256 12.5 / 16.7, 2.9e-7 / 1.4e-7;  512 x 512 x 512 21.5 / 26.7, 4.1e-7 / 1.5e-7;
+//   1024 x 1024 x 1024 40 / 44.5, 5.7e-7 / 1.6e-7
+// (512 tiles: 4096 x 1024 x 256 26 / 18; tiles cut short: 300 x 700 x 2048 94 / 86, at K = 64 8.7 / 9.2).
+// fp64-folded sums, whose fp32 kernel is slower, in one split, up to 64 tiles: the parallel backward
+// at T16 B16 D256 H32 33.5 / 37.1, T128 B1 D1024 H32 30.7 / 35.3, 2.0e-7 / 1.4e-7.
 bool stays_fp32(const GemmDesc& d, long s) {
-  if (d.N < 64) return d.acc64 ? (double)d.M * d.K < 6.5e6 : s < 2 || (double)d.M * d.K < 2e7;
   const bool whole_m = d.M % 128 == 0 || (d.M > 128 && d.K <= 64 && !d.acc64);
-  if (!vec_rows(d) || !whole_m || d.N % 64 || d.K % 32) return false;
+  if (s > 1 || !vec_rows(d) || !whole_m || d.N % 64 || d.K % 32) return false;
   const long tiles = tiles_of(d.M, d.N, 128, 64);
-  if (d.acc64) return s == 1 && tiles <= 64;
-  return tiles <= 256 && (s == 1 || (tiles > 128 && d.K < 1024));
+  return d.acc64 ? tiles <= 64 : tiles <= 256 && d.K <= 256;
 }
 int mid_take(const GemmDesc& d, long max_planes, int* mid) {
   if (!split_products_mode()) return 0;

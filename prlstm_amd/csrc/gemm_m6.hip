@@ -257,11 +257,15 @@ void m6_launch(M6Args& g, int splits, hipStream_t s) {
 }  // namespace
 
 int gemm_m6_splits(int M, int N, int K, int trans_a, int trans_b, int lda, int ldb) {
-  if ((trans_a && trans_b) || M < 64 || N <= 32 || K < 64) return 0;
-  // (32 or fewer columns measured no better on 128 x 32 tiles than on the fp32 kernel's 32 x 32:
-  // T512 B10 D32 H700 parallel step 169.8 against 166.5 us)
-  // a handful of tiles is all latency, and a slice of the fp32 kernel takes less of it
-  // (products of 128 x 128 x 256: the T128 B1 D256 H32 parallel step 43.2 us, here 47.5)
+  // Fewer than 64 columns stay on the fp32 kernel's 32 x 32 tiles, whose four waves cut K: a 128 x
+  // 64 tile would be half padding and wait out K alone (A B^T 1000 x 60 x 300 7 us, here 18; 256 x 33
+  // x 4096 51, 167; the parallel backward at T148 B3 D60 H122 45, 71), and its fp64-folded sums of
+  // 32 k are nearer to 64 bits (dW_ih 512 x 40 x 512 7.2e-8, here 1.46e-7), also where this kernel
+  // is the faster one (M K above 6e6: the backward at T4000 B4 D40 H1024 450 us, here 318)
+  if ((trans_a && trans_b) || M < 64 || N < 64 || K < 64) return 0;
+  // a handful of tiles is all latency: ragged products of 1e6 to 6e6 multiply-adds take 0.7 to 0.9
+  // of the fp32 kernel's 12 to 29 us here, those of 3e5 twice its 4 (whole ones: see stays_fp32 in
+  // gemm.hip).  The line is above where the gain begins.
   if ((double)M * N * K < 6e6) return 0;
   // operands are addressed as raw buffers with 32-bit offsets (a tile's rows may start past the end)
   const size_t a = (size_t)((trans_a ? K : M) + 256) * lda, b = (size_t)((trans_b ? N : K) + 256) * ldb;

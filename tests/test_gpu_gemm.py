@@ -239,8 +239,8 @@ def test_split_products_exact_on_representable_sums(dev, split_products, layout,
     assert torch.equal(c32, exact)
 
 
-MIDDLE = [(64, 96, 1024), (65, 1024, 95), (129, 1000, 65), (200, 64, 1931), (1000, 63, 20303), (333, 65, 700),
-          (1310, 33, 15431), (700, 650, 2603), (1027, 130, 64),            # gemm_m6.hip: edges of tiles and slices
+MIDDLE = [(64, 96, 1024), (65, 1024, 95), (129, 1000, 65), (200, 64, 1931), (1000, 67, 203), (333, 65, 700),
+          (131, 97, 1430), (700, 650, 2603), (1027, 130, 64),            # gemm_m6.hip: edges of tiles and slices
           (128, 128, 16384), (256, 384, 2560), (1024, 256, 1040)]          # whole 128 x 128 tiles
 LAYOUTS = [(0, 0), (0, 1), (1, 0)]
 
@@ -305,14 +305,14 @@ def test_deep_products_of_few_tiles_use_the_workspace(dev, split_products, M, N,
 
 
 @pytest.mark.parametrize("M,N,K,ta,tb,ws,fp32", [
-    (256, 512, 64, 0, 1, 0, True), (1024, 2048, 512, 0, 1, 0, True), (2100, 128, 64, 0, 1, 0, True),
-    (1024, 1024, 128, 1, 0, 1, True), (1024, 512, 256, 0, 0, 1, True), (2048, 1024, 512, 1, 0, 1, True),
-    (1000, 63, 203, 0, 1, 0, True), (2048, 33, 9000, 0, 1, 1, True), (2048, 33, 9800, 0, 1, 1, False),
+    (256, 512, 64, 0, 1, 0, True), (1024, 2048, 256, 0, 1, 0, True), (2100, 128, 64, 0, 1, 0, True),
+    (1024, 1024, 128, 1, 0, 1, True), (1024, 512, 256, 0, 0, 1, True),
+    (1000, 63, 203, 0, 1, 0, True), (2048, 33, 9800, 1, 0, 1, True), (2048, 64, 9800, 1, 0, 1, False),
     (4096, 1024, 256, 0, 1, 0, False), (300, 704, 2048, 0, 1, 0, False), (1024, 512, 512, 1, 0, 1, False),
-    (1024, 2048, 516, 0, 1, 0, False)])
+    (1024, 1024, 288, 0, 1, 0, False), (1024, 2048, 260, 0, 1, 0, False)])
 def test_which_whole_products_stay_on_the_fp32_kernel(dev, split_products, M, N, K, ta, tb, ws, fp32):
-    """Whole tiles of the fp32 kernel on at most one workgroup per CU, in one split, and products
-    of fewer than 64 columns that are not large run there with split products on too (the results
+    """Whole tiles of the fp32 kernel on at most one workgroup per CU, in one split of at most
+    256 k, and products of fewer than 64 columns run there with split products on too (the results
     are the same bits); their neighbours do not."""
     g = torch.Generator().manual_seed(K)
     a = torch.randn(*((K, M) if ta else (M, K)), generator=g).to(dev)
@@ -328,6 +328,7 @@ def test_which_whole_products_stay_on_the_fp32_kernel(dev, split_products, M, N,
 @pytest.mark.parametrize("T,B,D,H", [(256, 8, 128, 512),    # K = 2048 either way, whole tiles
                                      (256, 7, 100, 333),    # ragged
                                      (35, 20, 650, 650),    # dx over K = 2600
+                                     (128, 32, 50, 300),    # fewer than 64 columns: the fp32 kernel either way
                                      (128, 32, 256, 256)])  # dW_ih over K = 4096
 def test_middle_gradients_as_accurate_as_fp64_folded_sums(dev, split_products, T, B, D, H, mean):
     """The weight gradient and dx products of the backward: with split products off their fp32
