@@ -113,16 +113,20 @@ struct StreamLaunches {
   bool recorded;
 };
 // The streams whose launches may still run side by side: together at most the device's CUs (or
-// one stream), so few.  A process that uses one stream pays a lock and a comparison per call:
-// its event is recorded (0.75 us of the host, 1 us of the stream) when a second stream comes,
-// and after each of the kKeepRecording calls that follow such a change.
+// one stream), so few.  A process that uses one stream pays a lock and a comparison per call.
+// An event costs 0.75 us of the host and 1 us of the stream (3 after a graph), so it is recorded
+// when another stream comes, behind whatever its own stream holds by then; where streams take
+// turns, within kTurn calls, it is recorded right after each of the next kKeepRecording calls, so
+// that the others wait for the call alone.
 struct StreamOrder {
   std::mutex mu;
   std::vector<StreamLaunches> streams;
   std::vector<hipEvent_t> spare;
-  int recording = 0;
+  int recording = 0;    // calls whose event is still to be recorded at once
+  int since_turn = 0;   // calls since another stream's came
+  hipStream_t last = nullptr;
 };
-constexpr int kKeepRecording = 64;
+constexpr int kKeepRecording = 64, kTurn = 3;
 StreamOrder g_order[64];
 std::atomic<int> g_launched{0};  // hsl_launched_workgroups
 
@@ -161,10 +165,16 @@ LaunchOrder::LaunchOrder(int workgroups, hipStream_t stream) : stream_(stream) {
   }
   if (own >= 0 && others == 0) {
     o.streams[own].workgroups = std::max(o.streams[own].workgroups, workgroups);
+    ++o.since_turn;
     return;
   }
   if (capturing(stream)) return;
-  if (others > 0) o.recording = kKeepRecording;
+  if (others > 0 && stream != o.last) {
+    if (o.since_turn <= kTurn) o.recording = kKeepRecording;
+    o.since_turn = 0;
+  }
+  o.last = stream;
+  ++o.since_turn;
   if (others + workgroups > di.num_cus) {
     std::vector<StreamLaunches> left;
     for (StreamLaunches& e : o.streams) {

@@ -17,7 +17,6 @@ parameters' ``.grad`` point at the gradients of the mode just replayed, or are
 parallel mode), exactly as an eager step leaves them.
 """
 
-import contextlib
 import threading
 
 import torch
@@ -25,17 +24,6 @@ import torch
 from . import _lib
 
 _capture_lock = threading.Lock()  # one capture at a time counts the library's launches
-
-
-@contextlib.contextmanager
-def _replay_order(workgroups, device):
-    """Orders what is replayed inside with the persistent launches of this process's other
-    streams, as the library orders eager calls: `workgroups` of a launch wait for each other."""
-    _lib.call("hsl_replay_begin", workgroups, _lib.stream_of(device))
-    try:
-        yield
-    finally:
-        _lib.call("hsl_replay_end")
 
 
 class GraphedTrainStep:
@@ -82,6 +70,7 @@ class GraphedTrainStep:
                 out, (h_n, c_n) = m(self.static_x, self.hx)
                 torch.autograd.backward([out], [self.grad_out])
             workgroups = _lib.load().hsl_launched_workgroups(0)
+        self._ordered(workgroups, lambda: None)  # wait for the side stream here, not in the first replay
         grads = {n: p.grad for n, p in m.named_parameters()}
         # Only detached views of the static outputs are kept (same memory): the captured
         # autograd graph, and with it the parameters' AccumulateGrad nodes created on the
@@ -89,6 +78,18 @@ class GraphedTrainStep:
         # own nodes instead of reusing those (a stream mismatch torch warns about).
         self._graphs[mode] = (graph, out.detach(), h_n.detach(), c_n.detach(), grads, workgroups)
         del out, h_n, c_n
+
+    def _ordered(self, workgroups, replay):
+        """replay(), ordered with the persistent launches that this process has on other streams,
+        as the library orders eager calls: the replay's largest launch has `workgroups`."""
+        if not workgroups:  # no launch whose workgroups wait for each other
+            return replay()
+        lib = _lib.load()
+        lib.hsl_replay_begin(workgroups, torch._C._cuda_getCurrentRawStream(self.static_x.device.index))
+        try:
+            replay()
+        finally:
+            lib.hsl_replay_end()
 
     @property
     def graph(self):
@@ -106,11 +107,7 @@ class GraphedTrainStep:
         graph, out, h_n, c_n, grads, workgroups = self._graphs[mode]
         if x is not None:
             self.static_x.copy_(x)
-        if workgroups:
-            with _replay_order(workgroups, self.static_x.device):
-                graph.replay()
-        else:
-            graph.replay()
+        self._ordered(workgroups, graph.replay)
         for n, p in self.module.named_parameters():
             p.grad = grads[n]
         self.static_out, self.static_h_n, self.static_c_n = out, h_n, c_n
