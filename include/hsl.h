@@ -171,7 +171,8 @@ int hsl_rec_fwd(const float* x, const float* h0, const float* c0,
  * device memory (code under hipGraph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  No counterpart in the reference.  Its workspace is a static
  * scratch array of 4 MiB inside the library, one per device, held until the
- * process ends; the call allocates nothing (no hipMalloc, no events) and clears
+ * process ends; the call allocates nothing (no hipMalloc, and no event unless another
+ * stream's persistent call has to be ordered before it) and clears
  * the parts that must start empty with a fill kernel.  Shapes whose workspace
  * exceeds 4 MiB are rejected with HSL_ERR_UNSUPPORTED; the persistent path with
  * the input projection fused (H <= 512, D <= 256, D % 4 == 0, 16-byte aligned x,

@@ -242,19 +242,18 @@ struct X6Operand {
 // pieces 1 and 2 (zero for such values) are not issued.  Thread t loads rows
 // 4 (t / 16) .. +3 at k-row t % 16 (8 bytes); lanes t and t^1 swap two of those rows, so
 // the even lane writes rows 0-1 and the odd lane rows 2-3, each as a (k even, k odd) pair.
-template <bool FULL, int NSET = 1>
+// Whole tiles only.
+template <int NSET = 1>
 struct X6OperandB16 {
   static constexpr int kWrites = 2, kLoads = 1;
   const unsigned short* base;
-  int ld, rows, kend;
+  int ld;
   int r0q, k0;  // first row of the thread's quad, its k-row offset
   int so;
   u32x2 vv[NSET];  // rows 0-1 and rows 2-3 of the quad, two bf16 each
-  __device__ __forceinline__ void init(const float* b, int ld_, int r0, int rows_, int kbeg, int kend_) {
+  __device__ __forceinline__ void init(const float* b, int ld_, int r0, int, int kbeg, int) {
     base = reinterpret_cast<const unsigned short*>(b);
     ld = ld_;
-    rows = rows_;
-    kend = kend_;
     const int t = threadIdx.x, odd = t & 1;
     r0q = r0 + 4 * (t / 16);
     k0 = kbeg + t % 16;
@@ -264,20 +263,7 @@ struct X6OperandB16 {
   __device__ __forceinline__ void load(int slice) {
     u32x2& v = vv[SET];
     const int kk = k0 + slice * kBK;
-    if constexpr (FULL) {
-      v = *reinterpret_cast<const u32x2*>(base + (size_t)kk * ld + r0q);
-    } else {
-      const bool kok = kk < kend;
-      const unsigned short* kp = base + (size_t)(kok ? kk : kend - 1) * ld;  // a k-row that exists
-      unsigned e[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int rr = r0q + i;
-        const unsigned x = kp[rr < rows ? rr : rows - 1];
-        e[i] = (kok && rr < rows) ? x : 0u;
-      }
-      v = u32x2{e[0] | (e[1] << 16), e[2] | (e[3] << 16)};
-    }
+    v = *reinterpret_cast<const u32x2*>(base + (size_t)kk * ld + r0q);
   }
   template <int SET>
   __device__ __forceinline__ void store(unsigned short* p0) const {  // piece 0 only
@@ -302,7 +288,7 @@ __device__ __forceinline__ void x6_tile(const X6Args& g, int m0, int n0, unsigne
   // step, three to 2.42-2.43).  The projection shape has no registers to spare.
   constexpr int NSET = S::FOLD && S::BM == 256 ? 3 : 1;
   using OpA = X6Operand<FULL, AKC, S::BM, NSET>;
-  using OpB = std::conditional_t<BP == 1, X6OperandB16<FULL, NSET>, X6Operand<FULL, BKC, S::BN, NSET>>;
+  using OpB = std::conditional_t<BP == 1, X6OperandB16<NSET>, X6Operand<FULL, BKC, S::BN, NSET>>;
   constexpr int NPP = BP == 1 ? 3 : 6;  // piece products per k-step
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / S::WN, wn = wave % S::WN;
