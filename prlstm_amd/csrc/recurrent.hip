@@ -2318,6 +2318,7 @@ bool group_launches_pay(int T, int H, int groups, int launches, bool bwd) {
   return T >= std::max(1 << launches, std::min(64, groups * launches / 40));
 }
 
+constexpr int kAnySteps = 1 << 30;  // plans the launches whatever the sequence's length
 int plan_persistent(int T, int B, int H, int D, bool bwd, PersistentPlan* pl) {
   *pl = PersistentPlan{};
   const int mode = recurrent_path_mode();
@@ -2826,14 +2827,22 @@ int rec_fwd(const float* x, const float* h0, const float* c0, const float* w_ih,
   }
   PersistentPlan pl;
   WidePlan wp;
-  if (!per_step) HSL_CHECK(plan_persistent(T, B, H, D, false, &pl));
-  if (!per_step && !pl.ok) HSL_CHECK(plan_wide(T, B, H, false, &wp));
+  const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
+  FwdWs w;
+  size_t need = 0;
+  const auto plan = [&](int steps) -> int {
+    if (!per_step) HSL_CHECK(plan_persistent(steps, B, H, D, false, &pl));
+    if (!per_step && !pl.ok) HSL_CHECK(plan_wide(steps, B, H, false, &wp));
+    if (pl.XP && !x_aligned) pl.XP = false;  // the fused projection loads x in 16-byte pieces
+    need = carve_fwd(ws, ws_bytes, T, B, H, fwd_needs(pl, wp, x_aligned), &w);
+    return HSL_OK;
+  };
+  HSL_CHECK(plan(T));
+  // a workspace sized for a longer sequence may hold its launches' buffers and not the per-step
+  // path's, which few steps would take
+  if (ws && ws_bytes < need && !pl.ok && !wp.ok) HSL_CHECK(plan(kAnySteps));
   if (recurrent_path_mode() == 2 && !pl.ok && !wp.ok)
     return fail(HSL_ERR_UNSUPPORTED, "persistent path does not fit (B=%d H=%d)", B, H);
-  const bool x_aligned = reinterpret_cast<uintptr_t>(x) % 16 == 0;
-  if (pl.XP && !x_aligned) pl.XP = false;  // the fused projection loads x in 16-byte pieces
-  FwdWs w;
-  const size_t need = carve_fwd(ws, ws_bytes, T, B, H, fwd_needs(pl, wp, x_aligned), &w);
   if (!ws || ws_bytes < need)
     return fail(HSL_ERR_ARG, "hsl_rec_fwd: workspace %zu bytes, need %zu%s", ws_bytes, need,
                 pl.ok && !x_aligned ? " (x is not 16-byte aligned, so the input-gate buffer is needed)" : "");
@@ -3042,12 +3051,19 @@ int hsl_rec_bwd(const float* dout, const float* dh_n, const float* dc_n, const f
     return fail(HSL_ERR_ARG, "hsl_rec_bwd: null pointer");
   PersistentPlan pl;
   WidePlan wp;
-  if (T > 0 && B > 0 && H > 0) HSL_CHECK(plan_persistent(T, B, H, D, true, &pl));
-  if (T > 0 && B > 0 && H > 0 && !pl.ok) HSL_CHECK(plan_wide(T, B, H, true, &wp));
-  if (T > 0 && B > 0 && H > 0 && recurrent_path_mode() == 2 && !pl.ok && !wp.ok)
-    return fail(HSL_ERR_UNSUPPORTED, "persistent path does not fit (B=%d H=%d)", B, H);
   BwdWs w;
-  const size_t need = carve_bwd(ws, ws_bytes, T, B, D, H, bwd_needs(pl, wp, dx != nullptr), &w);
+  size_t need = 0;
+  const bool any = T > 0 && B > 0 && H > 0;
+  const auto plan = [&](int steps) -> int {
+    if (any) HSL_CHECK(plan_persistent(steps, B, H, D, true, &pl));
+    if (any && !pl.ok) HSL_CHECK(plan_wide(steps, B, H, true, &wp));
+    need = carve_bwd(ws, ws_bytes, T, B, D, H, bwd_needs(pl, wp, dx != nullptr), &w);
+    return HSL_OK;
+  };
+  HSL_CHECK(plan(T));
+  if (any && ws && ws_bytes < need && !pl.ok && !wp.ok) HSL_CHECK(plan(kAnySteps));  // as in the forward
+  if (any && recurrent_path_mode() == 2 && !pl.ok && !wp.ok)
+    return fail(HSL_ERR_UNSUPPORTED, "persistent path does not fit (B=%d H=%d)", B, H);
   if (!ws || ws_bytes < need) return fail(HSL_ERR_ARG, "hsl_rec_bwd: workspace %zu bytes, need %zu", ws_bytes, need);
   const int TB = T * B;
   const size_t plane = (size_t)B * H, plane4 = (size_t)B * 4 * H;

@@ -12,7 +12,7 @@ import torch
 from conftest import assert_parity
 from oracle import hsl_oracle as O
 import prlstm_amd
-from prlstm_amd import functional
+from prlstm_amd import _lib, functional
 
 pytestmark = pytest.mark.gpu
 
@@ -198,6 +198,37 @@ def test_short_sequences_take_the_faster_path(dev, T, B, H, fwd, bwd):
     wide kernels, 2 the launches over the batch)."""
     check(T, B, 16, H, dev, 0, a=[0.3, 0.5, 0.1, 0.2], with_hx=True, fwd_path=fwd)
     assert prlstm_amd.last_recurrent_path() == bwd
+
+
+@pytest.mark.parametrize("T,B,D,H,path", [(3, 64, 16, 512, 2), (2, 40, 16, 2000, 3)])
+def test_workspace_of_a_longer_sequence(dev, T, B, D, H, path):
+    """A workspace sized for 20 steps serves fewer of them, also where those would run per step
+    and its buffers are larger: the launches run then, forward and backward."""
+    print(f"workspace of a longer sequence T={T} B={B} H={H}", flush=True)
+    lib, P, s = _lib.load(), _lib.ptr, _lib.stream_of(dev)
+    torch.manual_seed(2)
+    m = prlstm_amd.HeadStartLSTM(D, H).to(dev)
+    x, dout = torch.randn(T, B, D, device=dev), torch.randn(T, B, H, device=dev)
+    out = m(x)[0]
+    assert prlstm_amd.last_recurrent_path() == 1
+    out.backward(dout)
+    n = lib.hsl_rec_fwd_ws_bytes(20, B, D, H)
+    assert n < lib.hsl_rec_fwd_ws_bytes(T, B, D, H)
+    w = [p.detach() for p in (m.weight_ih_l0, m.weight_hh_l0, m.bias_ih_l0, m.bias_hh_l0, m.a)]
+    h, c, act, tc = (torch.empty(*d, device=dev) for d in ((T + 1, B, H), (T + 1, B, H), (T, B, H, 4), (T, B, H)))
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    _lib.call("hsl_rec_fwd", P(x), None, None, *map(P, w), P(h), P(c), P(act), P(tc), P(ws), n, T, B, D, H, s)
+    assert prlstm_amd.last_recurrent_path() == path
+    assert (h[1:] - out).abs().max() < 1e-5
+    n = lib.hsl_rec_bwd_ws_bytes_for(20, B, D, H, 0)
+    ws = torch.empty(n, dtype=torch.uint8, device=dev)
+    g = [torch.empty_like(p) for p in w]
+    _lib.call("hsl_rec_bwd", P(dout), None, None, P(x), P(h), P(c), P(act), P(tc), P(w[0]), P(w[1]), P(w[3]), P(w[4]),
+              None, *map(P, g), None, None, P(ws), n, T, B, D, H, s)
+    torch.cuda.synchronize()
+    for got, p in zip(g, (m.weight_ih_l0, m.weight_hh_l0, m.bias_ih_l0, m.bias_hh_l0, m.a)):
+        assert float((got - p.grad).norm() / p.grad.norm()) < 1e-5
+    prlstm_amd.check_errors()
 
 
 def test_weight_gradient_of_several_launches_is_as_accurate_as_per_step(dev):
