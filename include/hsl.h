@@ -66,7 +66,8 @@ long long hsl_set_spin_timeout_us(long long us);
  * waits for the earlier one's call).  The replay of a graph that captured hsl_rec_fwd
  * or hsl_rec_bwd is ordered with them when it stands between the two calls below, on
  * the thread and stream that launch it (prlstm_amd.graph does so), with the workgroups
- * of its largest launch; the thread holds the library's launch lock between them.
+ * of its largest launch; the thread holds the library's launch lock between them, so
+ * other threads' calls wait for the end, and its own calls there are not ordered.
  * hsl_launched_workgroups gives the workgroups of the largest persistent launch of
  * this process since it was last called with clear != 0 (0: none, as in the per-step
  * path and the scans, which need no order).  Not ordered, and for the caller to

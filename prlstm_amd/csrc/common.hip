@@ -148,11 +148,15 @@ void record_launches(StreamOrder& o, StreamLaunches& e) {
 }
 }  // namespace
 
+namespace {
+thread_local LaunchOrder* g_replay = nullptr;  // between hsl_replay_begin and hsl_replay_end
+}
+
 LaunchOrder::LaunchOrder(int workgroups, hipStream_t stream) : stream_(stream) {
   for (int most = g_launched.load(); most < workgroups && !g_launched.compare_exchange_weak(most, workgroups);) {
   }
   DeviceInfo di;
-  if (device_info(&di) != HSL_OK) return;
+  if (g_replay || device_info(&di) != HSL_OK) return;  // (a replay's thread holds the lock)
   StreamOrder& o = g_order[di.device];
   o.mu.lock();
   device_ = di.device;
@@ -210,10 +214,6 @@ LaunchOrder::~LaunchOrder() {
       }
     }
   o.mu.unlock();
-}
-
-namespace {
-thread_local LaunchOrder* g_replay = nullptr;
 }
 
 int recurrent_path_mode() { return g_path_mode.load(); }

@@ -129,4 +129,6 @@ def test_replay_order_is_one_at_a_time(dev):
     assert lib.hsl_replay_end() == 1 and b"no hsl_replay_begin" in lib.hsl_last_error()
     assert lib.hsl_replay_begin(256, s) == 0
     assert lib.hsl_replay_begin(256, s) == 1 and b"not ended" in lib.hsl_last_error()
+    m, x = _module(dev, 16, 64), torch.randn(5, 4, 16, device=dev)
+    assert torch.isfinite(m(x)[0]).all()  # a call of the thread that holds the lock
     assert lib.hsl_replay_end() == 0
