@@ -2306,16 +2306,24 @@ constexpr int kMaxGroupLaunches = 4;
 // Whether T steps are enough for several launches.  Each starts by loading its W_hh registers
 // (4 to 10 us), and the backward ends by adding one dW_hh plane per group; per step they save
 // less the more of them there are.  Time of launches over time per step, D = 64, by T:
-//   forward, 2 launches: 0.66-0.83 at 4 (H = 450, 4-byte loads of W_hh: 1.36 at 2, 0.94 at 4);
-//     3: 0.86-1.11 at 4 (H = 450 1.31), 0.70-0.92 at 8;  4: 1.1-1.7 at 4, 0.91-1.27 at 8,
-//     0.75-1.00 at 16, except H = 512 B = 128: 1.08 at 16, 0.96 at 32
-//   backward, H >= 100, 2 launches: 0.55-0.99 at 4;  3: 0.84-1.22 at 4, 0.65-0.97 at 8;
-//     4: 0.97-1.18 at 8, 0.68-1.00 at 16;  small H, where a launch holds up to 256 groups:
-//     H = 16, 512 groups (2) 1.05 at 16, 0.77 at 32, 1024 (4) 1.19 at 32, 0.92 at 48;
-//     H = 32, 256 groups (2) 0.99 at 12, 512 (4) 1.11 at 32, 0.98 at 48;  H = 64, 256 (4) 1.00 at 16
+//   forward, 2 launches: H <= 384 0.73-0.98 at 2, H = 450 (4-byte loads of W_hh) and 512 1.01-1.36
+//     at 2, 0.79-0.96 at 4;  3: 0.86-1.11 at 4, 0.76-1.00 at 6 (H = 450 1.08, 0.92 at 8);  4: H = 100,
+//     200, 300 1.06-1.13 at 4, 0.91-0.96 at 8, H = 64, 128, 256, 384 1.02-1.17 at 8, 0.76-1.00 at 16,
+//     H = 450 1.19 at 8, 0.98 at 12, H = 512 1.08 at 16, 0.96 at 32
+//   backward, H >= 100, 2 launches: H <= 256 0.65-0.92 at 2, above 1.03-1.22 at 2, 0.80-0.99 at 4;  3:
+//     H <= 300 0.84-1.06 at 4, 0.72-0.94 at 6, above 0.89-1.07 at 6, 0.83-0.97 at 8;  4: H <= 256
+//     0.91-1.15 at 6, 0.83-1.03 at 8, above 1.01-1.10 at 12, 0.75-0.94 at 16
+//   backward at small H, where a launch holds up to 256 groups: H = 16, 512 groups (2) 1.05 at 16, 0.77
+//     at 32, 1024 (4) 1.19 at 32, 0.92 at 48;  H = 32, 256 groups (2) 0.99 at 12, 512 (4) 1.11 at 32,
+//     0.98 at 48;  H = 64, 256 (4) 1.00 at 16
 bool group_launches_pay(int T, int H, int groups, int launches, bool bwd) {
-  if (!bwd) return T >= (launches == 4 && H > 448 ? 24 : 1 << launches);
-  return T >= std::max(1 << launches, std::min(64, groups * launches / 40));
+  if (!bwd) {
+    if (launches == 2) return T >= (H > 384 ? 4 : 2);
+    if (launches == 3) return T >= (H > 448 && H % 4 ? 8 : 6);
+    return T >= (H > 448 ? (H % 4 ? 12 : 24) : H % 64 ? 8 : 16);
+  }
+  const int start = launches == 2 ? (H <= 256 ? 2 : 4) : launches == 3 ? (H <= 320 ? 6 : 8) : H <= 256 ? 8 : 16;
+  return T >= std::max(start, std::min(64, groups * launches / 40));
 }
 
 constexpr int kAnySteps = 1 << 30;  // plans the launches whatever the sequence's length
@@ -2445,25 +2453,34 @@ int wide_launches(int H) {
 // 64 MB of them, 15 to 40 us), which the widths' own sizes at one launch regain in the first
 // step.  Time of the wide kernels over time per step, D = 64, by T:
 //   512 < H <= 1024, one launch: forward 0.95 or less, backward 0.81-1.03 at 1;  two (H % 4 != 0):
-//     forward 0.79-1.12 at 2, 0.72-0.99 at 4, backward 0.91-1.03 at 4, 0.86-0.99 at 6
+//     H = 650 forward 1.12 at 2, 0.87-0.99 at 4, backward 1.03 at 4, 0.96-0.99 at 6;  H = 1023
+//     forward 1.08 at 1, 0.86-0.94 at 2, backward 1.02 at 2, 0.96 at 3
 //   1024 < H, one launch of at most 16 rows (B) or more: forward 1.04 or less at 1 (H < 1300 with
-//     B > 16: 1.10 at 1, 0.98 at 8);  backward B <= 16: H = 1100 1.12 at 4, 1.00 at 6, 1500 1.02
-//     at 3, 0.96 at 4, 1700 1.05 at 2, 0.96 at 3, 2000 1.05 at 1, 0.94 at 2;  B > 16: H = 1100 1.05 at 12, 1.00
-//     at 16, 1300 1.03 at 8, 0.96 at 12, 1500 1.06 at 4, 0.98 at 6, 1800 1.04 at 2, 0.95 at 4, 2000 0.99 at 2
-//   two to four launches: forward H = 1500 1.03 at 8, 0.98 at 12, 1700 to 2048 1.07 at 4,
-//     0.85-0.99 at 8;  backward H = 1500 1.02 at 12, 0.96 at 16, 1700 to 2000 two and three 0.82-0.99
-//     at 8, four 1.04 at 12, 0.98 at 16;  H = 2048 two 0.89 at 1, three 0.96 at 2, four 0.99 at 4
+//     B > 16: 1.10 at 1, 1.05 at 4, 1.00 at 6);  backward B <= 16: H = 1100 1.12 at 4, 1.00 at 6, 1500
+//     1.02 at 3, 0.96 at 4, 1700 1.05 at 2, 0.96 at 3, 2000 1.05 at 1, 0.94 at 2;  B > 16: H = 1100
+//     1.05 at 12, 1.00 at 16, 1300 1.03 at 8, 0.96 at 12, 1500 1.06 at 4, 0.98 at 6, 1800 1.04 at 2,
+//     0.95 at 4, 2000 0.99 at 2
+//   two launches: forward H = 1500 1.03 at 8, 0.98 at 12, 1700 1.03 at 4, 0.94 at 6, 1800 1.06 at 3,
+//     0.98 at 4, 2000 1.04 at 2, 0.93 at 4, 2048 B = 48 1.03 at 1, 0.97 at 2, B = 64 1.01 at 6, 0.97
+//     at 8;  backward H = 1500 1.02 at 12, 0.96 at 16, 1700 and 1800 1.04 at 6, 0.95 at 8, 2000 1.05 at
+//     4, 0.95 at 6, 2048 0.89 at 1
+//   three and four: forward H = 1800 1.03 at 6, 0.96 at 8, 2000 1.07 at 4, 0.97 at 6, 2048 three 1.05
+//     at 6, 0.99 at 8, four 1.09 at 4, 0.99 at 6;  backward three 1.08 at 6, 0.99 at 8 (2048: 0.96 at
+//     2), four 1.04 at 12, 0.98 at 16 (2048: 0.99 at 4)
 bool wide_pays(int T, int B, int H, int launches, bool bwd) {
-  if (H <= 1024) return launches == 1 || T >= (bwd ? 6 : 4);
+  if (H <= 1024) return launches == 1 || T >= (H < 900 ? (bwd ? 6 : 4) : (bwd ? 3 : 2));
   if (launches == 1) {
     if (H == 2048) return true;
-    if (!bwd) return B <= 16 || H >= 1300 || T >= 8;
+    if (!bwd) return B <= 16 || H >= 1300 || T >= 6;
     if (B <= 16) return T >= (H < 1350 ? 6 : H < 1600 ? 4 : H < 1900 ? 3 : 2);
     return T >= (H < 1250 ? 16 : H < 1350 ? 12 : H < 1600 ? 8 : H < 1900 ? 4 : 2);
   }
-  if (!bwd) return T >= (H < 1600 ? 12 : 8);
-  if (H == 2048) return T >= (launches == 4 ? 4 : launches == 3 ? 2 : 1);
-  return T >= (H < 1600 || launches == 4 ? 16 : 8);
+  if (bwd) {
+    if (H == 2048) return T >= (launches == 4 ? 4 : launches == 3 ? 2 : 1);
+    return T >= (H < 1600 || launches == 4 ? 16 : launches == 2 && H >= 1900 ? 6 : 8);
+  }
+  if (launches == 2) return T >= (H < 1600 ? 12 : H < 1750 ? 6 : H < 2048 ? 4 : B <= 48 ? 2 : 8);
+  return T >= (H < 1900 || (H == 2048 && launches == 3) ? 8 : 6);
 }
 
 int plan_wide(int T, int B, int H, bool bwd, WidePlan* pl) {

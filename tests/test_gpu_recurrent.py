@@ -186,11 +186,12 @@ def test_one_step_of_few_rows(dev, B, D, H, with_hx):
 
 
 @pytest.mark.parametrize("T,B,H,fwd,bwd", [
-    (3, 40, 260, 1, 1), (4, 40, 260, 2, 2), (7, 270, 128, 1, 1), (8, 270, 128, 2, 2),     # 2 and 3 launches
-    (15, 100, 300, 1, 1), (16, 100, 300, 2, 2), (16, 100, 450, 1, 2),                     # 4 launches
+    (1, 40, 260, 1, 1), (3, 40, 260, 2, 1), (4, 40, 260, 2, 2),                           # 2 launches
+    (5, 270, 128, 1, 1), (6, 270, 128, 2, 2),                                             # 3
+    (7, 100, 300, 1, 1), (15, 100, 300, 2, 1), (16, 100, 300, 2, 2), (11, 100, 450, 1, 1), (12, 100, 450, 2, 1),  # 4
     (6, 576, 32, 2, 1), (8, 576, 32, 2, 2),                                               # 144 groups
     (1, 9, 520, 3, 3), (4, 33, 650, 3, 1), (6, 33, 650, 3, 3),                            # width 1024
-    (1, 9, 1100, 3, 1), (6, 9, 1100, 3, 3), (7, 17, 1100, 1, 1), (8, 17, 1100, 3, 1),     # width 2048
+    (1, 9, 1100, 3, 1), (6, 9, 1100, 3, 3), (5, 17, 1100, 1, 1), (6, 17, 1100, 3, 1),     # width 2048
     (3, 9, 1500, 3, 1), (1, 9, 2000, 3, 1), (2, 17, 2000, 3, 3), (1, 40, 2048, 1, 3), (8, 40, 1800, 3, 3)])
 def test_short_sequences_take_the_faster_path(dev, T, B, H, fwd, bwd):
     """Several launches, and the wide kernels below their own widths, have to load W_hh first:

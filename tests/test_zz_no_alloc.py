@@ -136,9 +136,9 @@ def test_rec_fwd_noalloc_rejects_shapes_beyond_its_scratch(dev):
         assert torch.isnan(o[n]).all(), n
 
 
-@pytest.mark.parametrize("T,path", [(3, 1), (6, 2), (7, 1)])
+@pytest.mark.parametrize("T,path", [(1, 1), (6, 2), (7, 1)])
 def test_rec_fwd_noalloc_accepts_batches_of_several_launches(dev, T, path):
-    """B = 256 at H = 128 runs as two persistent launches (from 4 steps on), whose hand-off slots
+    """B = 256 at H = 128 runs as two persistent launches (from 2 steps on), whose hand-off slots
     (1 MiB) lie beside the gate buffer when D > 256.  Where both fit the scratch they run; at 7
     steps only the per-step path's buffers fit (3.94 MB of 4.19), which the call accepts as ever
     and runs; either way the outputs are those of hsl_rec_fwd on that path, bit for bit."""
