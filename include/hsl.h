@@ -74,7 +74,7 @@ long long hsl_set_spin_timeout_us(long long us);
  * keep apart: other replays, other processes on the device, and kernels of other
  * libraries that hold CUs while they wait (a collective whose peers come late).  A
  * launch that waits for its workgroups longer than the spin limit fails as described
- * there.  A stream is to be destroyed only when its calls have ended. */
+ * there.  Between the two calls the thread launches the replay and nothing else. */
 int hsl_launched_workgroups(int clear);
 int hsl_replay_begin(int workgroups, void* stream);
 int hsl_replay_end(void);

@@ -113,11 +113,12 @@ struct StreamLaunches {
   bool recorded;
 };
 // The streams whose launches may still run side by side: together at most the device's CUs (or
-// one stream), so few.  A process that uses one stream pays a lock and a comparison per call.
-// An event costs 0.75 us of the host and 1 us of the stream (3 after a graph), so it is recorded
-// when another stream comes, behind whatever its own stream holds by then; where streams take
-// turns, within kTurn calls, it is recorded right after each of the next kKeepRecording calls, so
-// that the others wait for the call alone.
+// one stream), so few.  A stream's event is recorded after each of its calls (0.75 us of the host,
+// 1 us of the stream, 3 after a graph): by the time another stream comes, the handle may be gone.
+// The default stream stays, so its event is recorded only when another stream comes, behind
+// whatever it holds by then, and a process that uses that stream alone pays a lock and a
+// comparison; where streams take turns, within kTurn calls, it too is recorded after each of the
+// next kKeepRecording calls, so that the others wait for the call alone.
 struct StreamOrder {
   std::mutex mu;
   std::vector<StreamLaunches> streams;
@@ -135,7 +136,7 @@ bool capturing(hipStream_t s) {
   return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
 }
 
-// Records e's event on its stream; not on one that is being captured or is gone.
+// Records e's event on its stream, unless that is being captured (a captured call has not run).
 void record_launches(StreamOrder& o, StreamLaunches& e) {
   if (capturing(e.stream)) return;
   if (!e.event && !o.spare.empty()) {
@@ -145,6 +146,7 @@ void record_launches(StreamOrder& o, StreamLaunches& e) {
   constexpr unsigned kFlags = hipEventDisableTiming | hipEventDisableSystemFence;  // order within the device only
   if (!e.event && hipEventCreateWithFlags(&e.event, kFlags) != hipSuccess) e.event = nullptr;
   e.recorded = e.event && hipEventRecord(e.event, e.stream) == hipSuccess;
+  if (!e.recorded) (void)hipGetLastError();  // an order that could not be had is no error of the call
 }
 }  // namespace
 
@@ -186,7 +188,7 @@ LaunchOrder::LaunchOrder(int workgroups, hipStream_t stream) : stream_(stream) {
         left.push_back(e);
         continue;
       }
-      if (!e.recorded) record_launches(o, e);
+      if (!e.recorded && !e.stream) record_launches(o, e);
       if (e.recorded) (void)hipStreamWaitEvent(stream, e.event, 0);
       if (e.event) o.spare.push_back(e.event);
     }
@@ -206,12 +208,12 @@ LaunchOrder::~LaunchOrder() {
   if (device_ < 0) return;
   StreamOrder& o = g_order[device_];
   for (StreamLaunches& e : o.streams)
-    if (e.stream == stream_ && !(e.recorded && capturing(stream_))) {  // (a captured call has not run)
-      e.recorded = false;
-      if (o.recording > 0) {
-        --o.recording;
+    if (e.stream == stream_) {
+      if (stream_ || o.recording > 0)
         record_launches(o, e);
-      }
+      else
+        e.recorded = false;
+      if (o.recording > 0) --o.recording;
     }
   o.mu.unlock();
 }
